@@ -265,6 +265,105 @@ int s2attn_permute_to_nchw(const void *src, void *dst, int64_t B, int64_t H, int
                            void *stream);
 
 /*
+ * The module's 1x1 projections (attention.py:519-571) between the NCHW tensors of a model and the NHWC tensors of the attention:
+ *   s2attn_proj_nchw_to_nhwc   dst_p[b, n, o] = sum_c src[b, c, n] W[o, c] + bias[o]; up to three destinations that share the
+ *                              source (q, k, v), each a packed [B, points, channels] tensor; also dy W of the output projection
+ *   s2attn_proj_nhwc_to_nchw   dst[b, o, n] = sum over sources and their channels of W[o, c] src_p[b, n, c] + bias[o]: the output
+ *                              projection, and the input gradient of the projections (three sources: dq, dk, dv)
+ *   s2attn_grad_partials       partial sums over slices of the points of sum_n pm_p[n, j] cm[i, n] (weight gradients) and of both
+ *                              operands alone (bias gradients)
+ * Element type of the arithmetic (`compute`): S2ATTN_F32 takes fp32 tensors (products of three-term bf16 splits, fp32
+ * accumulation: as exact as fp32 multiply-adds), S2ATTN_BF16 / S2ATTN_F16 16-bit ones, or an fp32 NCHW tensor that is rounded on
+ * the way in (autocast) and its fp32 gradient.
+ *
+ * Weights are packed once per call (s2attn_pack_weights) into blocks of 64 rows x 16 columns in the order the kernels take:
+ * a job lays one matrix, element (r, c) at w[r * row_stride + c * col_stride], times scale, at rows 64 * first_block and
+ * columns 16 * first_k16 of a packed array of total_k16 column groups, and its bias times scale (zeros without one) at
+ * dst_bias[64 * first_block] (unless null).  Matrices that share rows (one destination, several sources) lie next to
+ * each other along the columns, s2attn_pack_k16(cols) groups each; matrices that share columns (several destinations) below
+ * each other, (rows + 63) / 64 blocks each.  The array is s2attn_pack_bytes(blocks, k16) long and 16-byte aligned.
+ */
+#define S2ATTN_PROJ_MAX_PARTS 3
+#define S2ATTN_PACK_MAX_JOBS 8
+#define S2ATTN_FINISH_MAX_JOBS 10
+
+typedef struct s2attn_pack_job {
+    const void *w, *bias;
+    void *dst;
+    float *dst_bias;
+    int64_t row_stride, col_stride;
+    int rows, cols, dtype;
+    int first_block, first_k16, total_k16;
+    float scale;
+} s2attn_pack_job;
+
+int s2attn_pack_k16(int cols, int compute);
+int64_t s2attn_pack_bytes(int blocks, int k16, int compute);
+int s2attn_pack_weights(const s2attn_pack_job *jobs, int njobs, int compute, void *stream);
+
+typedef struct s2attn_proj {
+    int batch;
+    int nsrc, ndst; /* one source (nchw_to_nhwc) or one destination (nhwc_to_nchw) */
+    int src_dtype, dst_dtype, compute;
+    int64_t points; /* grid points of one batch element */
+    const void *src[S2ATTN_PROJ_MAX_PARTS];
+    void *dst[S2ATTN_PROJ_MAX_PARTS];
+    int src_channels[S2ATTN_PROJ_MAX_PARTS], dst_channels[S2ATTN_PROJ_MAX_PARTS];
+    const void *packed;
+    const float *bias; /* of the packed blocks, or null */
+} s2attn_proj;
+
+int s2attn_proj_nchw_to_nhwc(const s2attn_proj *p, void *stream);
+int s2attn_proj_nhwc_to_nchw(const s2attn_proj *p, void *stream);
+
+typedef struct s2attn_grad {
+    int batch, npm;
+    int cm_dtype, pm_dtype, compute;
+    int cm_channels, pm_channels[S2ATTN_PROJ_MAX_PARTS];
+    int64_t points;
+    const void *cm;                        /* [B, cm_channels, points] */
+    const void *pm[S2ATTN_PROJ_MAX_PARTS]; /* [B, points, pm_channels] */
+    float *part;                           /* [slices][sum of pm_channels][cm_channels] */
+    float *part_cm;                        /* [slices][cm_channels] sums of cm over the points, or null */
+    float *part_pm;                        /* [slices][sum of pm_channels] sums of pm, or null */
+} s2attn_grad;
+
+int s2attn_grad_slices(const s2attn_grad *g); /* slices of this problem, or a negative error */
+int s2attn_grad_partials(const s2attn_grad *g, void *stream);
+
+/* out[r * row_stride + c * col_stride] = scale * sum over slices of part[slice * slice_stride + r * cols + c], in slice order
+ * independent of the launch: results are the same in every run. */
+typedef struct s2attn_finish_job {
+    const float *part;
+    void *out;
+    int64_t slice_stride, row_stride, col_stride;
+    int slices, rows, cols, dtype;
+    float scale;
+} s2attn_finish_job;
+
+int s2attn_finish(const s2attn_finish_job *jobs, int njobs, void *stream);
+
+/*
+ * RMS norm over the channels of a head (attention.py:540-549): y = x rsqrt(mean(x^2) + eps) (1 + gain) mult, for up to two tensors
+ * (q and k) of rows = points x heads contiguous rows of head_channels values.  The backward takes x and, in y, the gradient of
+ * the result, which it replaces by the gradient of x; dgain[blocks][head_channels] receives partial sums of the gradient of
+ * gain / mult (add them with s2attn_finish, scale = mult).
+ */
+typedef struct s2attn_norm {
+    int ntensors, head_channels, dtype, gain_dtype, blocks;
+    float eps;
+    const void *x[2];
+    void *y[2];
+    const void *gain[2];
+    float *dgain[2];
+    int64_t rows[2];
+    float mult[2];
+} s2attn_norm;
+
+int s2attn_head_norm(const s2attn_norm *n, void *stream);
+int s2attn_head_norm_backward(const s2attn_norm *n, void *stream);
+
+/*
  * Ring-step variants of the gather direction (nlon_in a multiple of nlon_out): the pieces a longitude-sharded layer is
  * built from.  K/V arrive one longitude chunk at a time (in such a layer the chunks travel around a ring of devices);
  * q, dy and the per-point softmax state stay with the caller.  Each call handles ONE chunk on ONE device and talks to

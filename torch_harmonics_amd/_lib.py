@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(_HERE, "libs2attn.so")
 TORCH_LIB_PATH = os.path.join(_HERE, "_C.so")  # libtorch registration of the operators (csrc/s2attn_torch.cpp)
 
 S2ATTN_F32, S2ATTN_BF16, S2ATTN_F16 = 0, 1, 2
-ABI_VERSION = 12
+ABI_VERSION = 13
 NOALLOC_SCRATCH_BYTES = 64 * 1024 * 1024
 
 _vp = ctypes.c_void_p
@@ -63,6 +63,40 @@ class ShapeStruct(ctypes.Structure):
     ]  # fmt: skip
 
 
+PROJ_MAX_PARTS = 3
+
+
+class PackJobStruct(ctypes.Structure):
+    _fields_ = [("w", _vp), ("bias", _vp), ("dst", _vp), ("dst_bias", _vp), ("row_stride", _i64), ("col_stride", _i64)] + [
+        (n, _int) for n in ("rows", "cols", "dtype", "first_block", "first_k16", "total_k16")
+    ] + [("scale", ctypes.c_float)]  # fmt: skip
+
+
+class ProjStruct(ctypes.Structure):
+    _fields_ = [(n, _int) for n in ("batch", "nsrc", "ndst", "src_dtype", "dst_dtype", "compute")] + [
+        ("points", _i64), ("src", _vp * PROJ_MAX_PARTS), ("dst", _vp * PROJ_MAX_PARTS),
+        ("src_channels", _int * PROJ_MAX_PARTS), ("dst_channels", _int * PROJ_MAX_PARTS), ("packed", _vp), ("bias", _vp),
+    ]  # fmt: skip
+
+
+class GradStruct(ctypes.Structure):
+    _fields_ = [(n, _int) for n in ("batch", "npm", "cm_dtype", "pm_dtype", "compute", "cm_channels")] + [
+        ("pm_channels", _int * PROJ_MAX_PARTS), ("points", _i64), ("cm", _vp), ("pm", _vp * PROJ_MAX_PARTS), ("part", _vp), ("part_cm", _vp), ("part_pm", _vp),
+    ]  # fmt: skip
+
+
+class FinishJobStruct(ctypes.Structure):
+    _fields_ = [("part", _vp), ("out", _vp), ("slice_stride", _i64), ("row_stride", _i64), ("col_stride", _i64)] + [
+        (n, _int) for n in ("slices", "rows", "cols", "dtype")
+    ] + [("scale", ctypes.c_float)]  # fmt: skip
+
+
+class NormStruct(ctypes.Structure):
+    _fields_ = [(n, _int) for n in ("ntensors", "head_channels", "dtype", "gain_dtype", "blocks")] + [
+        ("eps", ctypes.c_float), ("x", _vp * 2), ("y", _vp * 2), ("gain", _vp * 2), ("dgain", _vp * 2), ("rows", _i64 * 2), ("mult", ctypes.c_float * 2),
+    ]  # fmt: skip
+
+
 class RingShapeStruct(ctypes.Structure):
     _fields_ = [
         ("batch", ctypes.c_int32),
@@ -106,6 +140,16 @@ SYMBOLS = {
     "s2attn_backward_dkdv": (_int, [_vp] * 8 + [ctypes.POINTER(PlanStruct), ctypes.POINTER(ShapeStruct), _vp]),
     "s2attn_permute_to_nhwc": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
     "s2attn_permute_to_nchw": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
+    "s2attn_pack_k16": (_int, [_int, _int]),
+    "s2attn_pack_bytes": (_i64, [_int, _int, _int]),
+    "s2attn_pack_weights": (_int, [ctypes.POINTER(PackJobStruct), _int, _int, _vp]),
+    "s2attn_proj_nchw_to_nhwc": (_int, [ctypes.POINTER(ProjStruct), _vp]),
+    "s2attn_proj_nhwc_to_nchw": (_int, [ctypes.POINTER(ProjStruct), _vp]),
+    "s2attn_grad_slices": (_int, [ctypes.POINTER(GradStruct)]),
+    "s2attn_grad_partials": (_int, [ctypes.POINTER(GradStruct), _vp]),
+    "s2attn_finish": (_int, [ctypes.POINTER(FinishJobStruct), _int, _vp]),
+    "s2attn_head_norm": (_int, [ctypes.POINTER(NormStruct), _vp]),
+    "s2attn_head_norm_backward": (_int, [ctypes.POINTER(NormStruct), _vp]),
     "s2attn_ring_forward_step": (_int, [_vp] * 10 + [ctypes.POINTER(RingShapeStruct), _vp]),
     "s2attn_ring_forward_step_plan": (_int, [_vp] * 7 + [ctypes.POINTER(PlanStruct), ctypes.POINTER(RingShapeStruct), _vp]),
     "s2attn_ring_backward_pass1_plan": (_int, [_vp] * 10 + [ctypes.POINTER(PlanStruct), ctypes.POINTER(RingShapeStruct), _vp]),

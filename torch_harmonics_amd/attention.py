@@ -17,11 +17,14 @@ import torch.nn.functional as F
 from ._attention_utils import _check_dtypes_match, _check_extent, _check_ndim
 from ._layout import to_nchw, to_nhwc
 from .neighborhood import precompute_neighborhood_s2
-from .ops import neighborhood_s2_attention, takes_column_blocks
+from .ops import module_attention, module_attention_traced, neighborhood_s2_attention, takes_column_blocks
 from .plan import cached_host_blob
 from .quadrature import precompute_latitudes
 
 __all__ = ["NeighborhoodAttentionS2"]
+
+_PLAIN = (torch.Tensor, nn.Parameter)  # no subclass: those have behavior of their own, operator by operator
+_NATIVE = (torch.float32, torch.bfloat16, torch.float16)
 
 
 def _weight_grad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
@@ -435,6 +438,30 @@ class NeighborhoodAttentionS2(nn.Module):
         x = F.rms_norm(x, normalized_shape=gain.shape, weight=1 + gain if scale is None else (1 + gain) * scale)
         return x.reshape(B, H, W, C)
 
+    def _native_dtype(self, query, key, value) -> Optional[torch.dtype]:
+        """Element type in which the layer runs as one native operator, None where it is composed of separate operators instead: with a
+        tensor as softmax scale or another attention_handle, for fp64, for tensors that are not plain GPU tensors, and for mixtures
+        of types that torch itself would refuse."""
+        if self.attention_handle is not neighborhood_s2_attention or not isinstance(self.scale, (int, float)):
+            return None
+        dev, dtype, wdtype = query.device, query.dtype, self.q_weights.dtype
+        for t in (query, key, value):
+            if type(t) not in _PLAIN or t.device != dev or t.shape[0] != query.shape[0] or t.shape[1] != self.in_channels:
+                return None
+        if dev.type != "cuda" or query.numel() == 0 or wdtype not in _NATIVE:
+            return None
+        params = (self.q_weights, self.k_weights, self.v_weights, self.proj_weights, self.q_bias, self.k_bias, self.v_bias, self.proj_bias, self.q_norm_weights, self.k_norm_weights)
+        for p in params:
+            if p is not None and (type(p) not in _PLAIN or p.dtype != wdtype or p.device != dev):
+                return None
+        if self.psi_plan.device != dev or self.quad_weights.device != dev or self.psi_col_idx.device != dev:
+            return None
+        compute = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else wdtype
+        # outside autocast everything has one type; inside, an fp32 input is rounded on the way in like every operand
+        if compute not in _NATIVE or (dtype != compute and (dtype != torch.float32 or not torch.is_autocast_enabled("cuda"))):
+            return None
+        return compute
+
     def forward(self, query: torch.Tensor, key: Optional[torch.Tensor] = None, value: Optional[torch.Tensor] = None) -> torch.Tensor:
         """
         query : (B, in_channels, nlat_out, nlon_out); key, value : (B, in_channels, nlat_in, nlon_in), both
@@ -457,6 +484,15 @@ class NeighborhoodAttentionS2(nn.Module):
         _check_extent(value, -1, self.nlon_in, "value longitudes")
 
         key_is_query, value_is_query, value_is_key = key is query, value is query, value is key
+        compute = self._native_dtype(query, key, value)
+        if compute is not None:
+            layer = module_attention_traced if torch.compiler.is_compiling() else module_attention
+            return layer(
+                query, None if key_is_query else key, None if value_is_key else value,
+                self.q_weights, self.k_weights, self.v_weights, self.proj_weights, self.q_bias, self.k_bias, self.v_bias, self.proj_bias,
+                self.q_norm_weights, self.k_norm_weights, self.scale, self.quad_weights, self.psi_col_idx, self.psi_roff_idx, self.psi_plan, self._psi_plan_header,
+                self.num_heads, self.nlat_in, self.nlon_in, self.nlat_out, self.nlon_out, compute,
+            )  # fmt: skip
         # the softmax scale rides on the q projection (or on the q gain when the q/k RMS norm is on): no pass of its own
         normed = self.q_norm_weights is not None
         wq = self.q_weights.view(self.q_weights.shape[0], -1)

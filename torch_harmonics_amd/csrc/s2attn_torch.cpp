@@ -6,16 +6,24 @@
 // 553-570 and attention_cuda_bwd.cu:874-893), output allocation, the plan cache, and one call into the C ABI on torch's
 // current stream.  There is no CPU implementation: CPU tensors are refused with a clear error.
 //
+// s2attn_kernels::module_attention is the whole NeighborhoodAttentionS2 layer (projections, q/k norm, attention, output projection)
+// as ONE autograd node: eleven launches per training step and no Python between them, where the operator-by-operator form
+// needs about forty and spends 0.8 ms of host time on them.
+//
 // Built by the Makefile next to it into torch_harmonics_amd/_C.so and loaded with torch.ops.load_library; the fake (meta)
 // kernels and the autograd rules are registered from Python (torch_harmonics_amd/ops.py), as the reference does.
 
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/custom_class.h>
 #include <torch/library.h>
 
+#include <array>
 #include <list>
 #include <mutex>
+#include <string>
 #include <utility>
 #include <tuple>
 #include <vector>
@@ -306,6 +314,433 @@ std::tuple<Tensor, Tensor, Tensor> backward_saved(const Tensor &kx, const Tensor
     return backward_impl(kx, vx, qy, dy, &y, &lse, quad_weights, col_idx, row_off, num_heads, nlon_in, nlat_out, nlon_out, plan, plan_header);
 }
 
+// ---- the module as one autograd node ----------------------------------------------------------------------------------------
+struct LayerConfig {
+    int64_t num_heads = 1, nlat_in = 0, nlon_in = 0, nlat_out = 0, nlon_out = 0;
+    double scale = 1.0;
+    at::ScalarType compute = at::kFloat; // element type of q, k, v, y and of the result
+    std::vector<int64_t> plan_header;
+};
+
+constexpr float RMS_EPS = 1.1920928955078125e-7f; // F.rms_norm's default: the fp32 machine epsilon, for 16-bit inputs too
+
+int blocks64(int64_t c) { return (int)((c + 63) / 64); }
+void *at_byte(const Tensor &t, int64_t ofs) { return static_cast<char *>(t.data_ptr()) + ofs; }
+
+// Packed weights of several matrices in one allocation (see include/s2attn.h).
+struct Packer {
+    int compute;
+    std::vector<s2attn_pack_job> jobs;
+    std::vector<int64_t> at; // byte offsets of weights and bias inside the allocation, per job
+    int64_t bytes = 0;
+    explicit Packer(int c) : compute(c) {}
+    int k16(int64_t cols) const { return s2attn_pack_k16((int)cols, compute); }
+    int64_t reserve(int blocks, int k16s)
+    {
+        const int64_t o = bytes;
+        bytes += (s2attn_pack_bytes(blocks, k16s, compute) + 255) / 256 * 256;
+        return o;
+    }
+    int64_t reserve_bias(int blocks)
+    {
+        const int64_t o = bytes;
+        bytes += (int64_t)blocks * 256;
+        return o;
+    }
+    // w: [rows, cols] or, transposed, [cols, rows]
+    void add(const Tensor &w, const Tensor &bias, int64_t rows, int64_t cols, bool transposed, double scale, int64_t ofs, int64_t bias_ofs, int block, int first_k16, int total_k16)
+    {
+        s2attn_pack_job j = {};
+        j.w = w.data_ptr(), j.bias = bias.defined() ? bias.data_ptr() : nullptr;
+        j.rows = (int)rows, j.cols = (int)cols, j.dtype = dtype_code(w.scalar_type());
+        j.row_stride = transposed ? 1 : cols, j.col_stride = transposed ? rows : 1;
+        j.first_block = block, j.first_k16 = first_k16, j.total_k16 = total_k16, j.scale = (float)scale;
+        jobs.push_back(j), at.push_back(ofs), at.push_back(bias_ofs);
+    }
+    Tensor run(const Tensor &like, void *stream)
+    {
+        Tensor buf = at::empty({bytes}, like.options().dtype(at::kByte));
+        for (size_t i = 0; i < jobs.size(); i++) {
+            jobs[i].dst = at_byte(buf, at[2 * i]);
+            jobs[i].dst_bias = at[2 * i + 1] >= 0 ? static_cast<float *>(at_byte(buf, at[2 * i + 1])) : nullptr;
+        }
+        check_rc(s2attn_pack_weights(jobs.data(), (int)jobs.size(), compute, stream), "s2attn_pack_weights");
+        return buf;
+    }
+};
+
+struct Part {
+    const Tensor *t;
+    int64_t channels;
+};
+
+// One projection launch: NCHW source -> NHWC destinations (to_nhwc) or NHWC sources -> NCHW destination.
+void project(bool to_nhwc, const std::vector<Part> &src, const std::vector<Part> &dst, int64_t batch, int64_t points, int compute, const void *packed,
+             const void *bias, void *stream)
+{
+    s2attn_proj p = {};
+    p.batch = (int)batch, p.points = points, p.nsrc = (int)src.size(), p.ndst = (int)dst.size();
+    p.src_dtype = dtype_code(src[0].t->scalar_type()), p.dst_dtype = dtype_code(dst[0].t->scalar_type()), p.compute = compute;
+    for (size_t i = 0; i < src.size(); i++) p.src[i] = src[i].t->data_ptr(), p.src_channels[i] = (int)src[i].channels;
+    for (size_t i = 0; i < dst.size(); i++) p.dst[i] = dst[i].t->data_ptr(), p.dst_channels[i] = (int)dst[i].channels;
+    p.packed = packed, p.bias = static_cast<const float *>(bias);
+    check_rc(to_nhwc ? s2attn_proj_nchw_to_nhwc(&p, stream) : s2attn_proj_nhwc_to_nchw(&p, stream), "s2attn_proj");
+}
+
+// Weight and bias gradients: partial sums now, all final sums of the backward in one launch at its end.
+struct Gradients {
+    void *stream;
+    std::vector<s2attn_finish_job> jobs;
+    std::vector<Tensor> keep;
+    void job(const float *part, Tensor &out, int64_t slices, int64_t slice_stride, int64_t rows, int64_t cols, int64_t rs, int64_t cs, double scale)
+    {
+        s2attn_finish_job j = {};
+        j.part = part, j.out = out.data_ptr(), j.slice_stride = slice_stride, j.row_stride = rs, j.col_stride = cs;
+        j.slices = (int)slices, j.rows = (int)rows, j.cols = (int)cols, j.dtype = dtype_code(out.scalar_type()), j.scale = (float)scale;
+        jobs.push_back(j);
+    }
+    // cm [B, ci, points], pm_p [B, points, c_p]; returns the partials of pm x cm, pm and cm (the latter two undefined if not wanted)
+    std::tuple<Tensor, Tensor, Tensor, int64_t> partials(const Tensor &cm, int64_t ci, const std::vector<Part> &pm, int64_t batch, int64_t points, int compute, bool want_cm, bool want_pm)
+    {
+        s2attn_grad g = {};
+        g.batch = (int)batch, g.points = points, g.npm = (int)pm.size(), g.compute = compute;
+        g.cm = cm.data_ptr(), g.cm_channels = (int)ci, g.cm_dtype = dtype_code(cm.scalar_type()), g.pm_dtype = dtype_code(pm[0].t->scalar_type());
+        int64_t cj = 0;
+        for (size_t i = 0; i < pm.size(); i++) g.pm[i] = pm[i].t->data_ptr(), g.pm_channels[i] = (int)pm[i].channels, cj += pm[i].channels;
+        const int64_t slices = s2attn_grad_slices(&g);
+        check_rc(slices, "s2attn_grad_slices");
+        const auto opt = cm.options().dtype(at::kFloat);
+        Tensor part = at::empty({slices * cj * ci}, opt), sc, sp;
+        if (want_cm) sc = at::empty({slices * ci}, opt);
+        if (want_pm) sp = at::empty({slices * cj}, opt);
+        g.part = part.data_ptr<float>(), g.part_cm = want_cm ? sc.data_ptr<float>() : nullptr, g.part_pm = want_pm ? sp.data_ptr<float>() : nullptr;
+        check_rc(s2attn_grad_partials(&g, stream), "s2attn_grad_partials");
+        keep.push_back(part), keep.push_back(sc), keep.push_back(sp);
+        return {part, sc, sp, slices};
+    }
+    void finish()
+    {
+        if (!jobs.empty()) check_rc(s2attn_finish(jobs.data(), (int)jobs.size(), stream), "s2attn_finish");
+    }
+};
+
+Tensor dense(const Tensor &t) { return t.defined() ? t.contiguous() : t; }
+
+// Tensor arguments of the layer
+enum { XQ, XK, XV, WQ, WK, WV, WP, BQ, BK, BV, BP, NQ, NK, QUAD, COL, ROW, PLAN, NTENSORS };
+
+struct LayerState : torch::CustomClassHolder {
+    LayerConfig cfg;
+    int slot[NTENSORS]; // position among the tensors given to the node, -1: absent
+};
+
+// Which of q, k, v are made from an input: query (B, C, nlat_out, nlon_out), key and value (B, C, nlat_in, nlon_in); an absent
+// key is the query, an absent value the key.
+struct Source {
+    int x;             // XQ, XK or XV
+    int first, count;  // of q (0), k (1), v (2)
+};
+std::vector<Source> sources(bool has_key, bool has_value)
+{
+    if (!has_key) return has_value ? std::vector<Source>{{XQ, 0, 2}, {XV, 2, 1}} : std::vector<Source>{{XQ, 0, 3}};
+    return has_value ? std::vector<Source>{{XQ, 0, 1}, {XK, 1, 1}, {XV, 2, 1}} : std::vector<Source>{{XQ, 0, 1}, {XK, 1, 2}};
+}
+
+// Kept for the backward: the inputs (NCHW, as they came), q, k, v (and q, k before their norm), y and the softmax normaliser.
+enum { S_Q = NTENSORS, S_K, S_V, S_QRAW, S_KRAW, S_Y, S_LSE, NSAVED };
+
+constexpr int NKEPT = NSAVED - NTENSORS;
+constexpr int NGRADS = NK + 1; // tensor arguments that may need a gradient
+
+// The result, and in kept[] what S_Q ... S_LSE name (undefined where there is none; nothing without `keep`).
+Tensor layer_forward(const Tensor (&given)[NTENSORS], const LayerConfig &cfg, bool keep, Tensor (&kept)[NKEPT])
+{
+    Tensor t[NTENSORS];
+    for (int i = 0; i < NTENSORS; i++)
+        if (given[i].defined()) t[i] = given[i].contiguous();
+    const int64_t B = t[XQ].size(0), C = t[XQ].size(1), nh = cfg.num_heads, Ck = t[WQ].size(0), Cv = t[WV].size(0);
+    const int64_t Po = cfg.nlat_out * cfg.nlon_out, Pi = cfg.nlat_in * cfg.nlon_in;
+    const bool normed = t[NQ].defined();
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(t[XQ].device());
+    void *stream = current_stream(t[XQ].device());
+    const auto opt = t[XQ].options().dtype(cfg.compute);
+    const int comp = dtype_code(cfg.compute);
+
+    // weights in operand order: q | k | v below each other, and the output projection
+    Packer pk(comp);
+    const int64_t ch[3] = {Ck, Ck, Cv};
+    const int kin = pk.k16(C), first[4] = {0, blocks64(Ck), 2 * blocks64(Ck), 2 * blocks64(Ck) + blocks64(Cv)};
+    const int64_t w_ofs = pk.reserve(first[3], kin), b_ofs = t[BQ].defined() ? pk.reserve_bias(first[3]) : -1;
+    for (int i = 0; i < 3; i++) pk.add(t[WQ + i], t[BQ + i], ch[i], C, false, i == 0 && !normed ? cfg.scale : 1.0, w_ofs, b_ofs, first[i], 0, kin);
+    const int64_t p_ofs = pk.reserve(blocks64(Cv), pk.k16(Cv)), pb_ofs = t[BP].defined() ? pk.reserve_bias(blocks64(Cv)) : -1;
+    pk.add(t[WP], t[BP], Cv, Cv, false, 1.0, p_ofs, pb_ofs, 0, 0, pk.k16(Cv));
+    const Tensor packed = pk.run(t[XQ], stream);
+
+    Tensor qkv[3] = {at::empty({B, cfg.nlat_out, cfg.nlon_out, Ck}, opt), at::empty({B, cfg.nlat_in, cfg.nlon_in, Ck}, opt),
+                     at::empty({B, cfg.nlat_in, cfg.nlon_in, Cv}, opt)};
+    const int64_t block_bytes = s2attn_pack_bytes(1, kin, comp);
+    for (const Source &s : sources(t[XK].defined(), t[XV].defined())) {
+        std::vector<Part> dst;
+        for (int i = s.first; i < s.first + s.count; i++) dst.push_back({&qkv[i], ch[i]});
+        project(true, {{&t[s.x], C}}, dst, B, s.x == XQ ? Po : Pi, comp, at_byte(packed, w_ofs + first[s.first] * block_bytes),
+                b_ofs >= 0 ? at_byte(packed, b_ofs + first[s.first] * 256) : nullptr, stream);
+    }
+    Tensor raw[2];
+    if (normed) {
+        s2attn_norm n = {};
+        n.ntensors = 2, n.head_channels = (int)(Ck / nh), n.dtype = comp, n.gain_dtype = dtype_code(t[NQ].scalar_type()), n.eps = RMS_EPS;
+        n.blocks = 2048;
+        for (int i = 0; i < 2; i++) {
+            raw[i] = qkv[i];
+            if (keep) qkv[i] = at::empty_like(raw[i]); // else in place
+            n.x[i] = raw[i].data_ptr(), n.y[i] = qkv[i].data_ptr(), n.gain[i] = t[NQ + i].data_ptr(), n.mult[i] = i ? 1.f : (float)cfg.scale;
+            n.rows[i] = B * (i ? Pi : Po) * nh;
+        }
+        check_rc(s2attn_head_norm(&n, stream), "s2attn_head_norm");
+    }
+
+    auto [y, lse] = forward_impl(qkv[1], qkv[2], qkv[0], t[QUAD], t[COL], t[ROW], nh, cfg.nlon_in, cfg.nlat_out, cfg.nlon_out, keep, t[PLAN],
+                                 c10::OptionalArrayRef<int64_t>(cfg.plan_header));
+    Tensor out = at::empty({B, Cv, cfg.nlat_out, cfg.nlon_out}, opt);
+    project(false, {{&y, Cv}}, {{&out, Cv}}, B, Po, comp, at_byte(packed, p_ofs), pb_ofs >= 0 ? at_byte(packed, pb_ofs) : nullptr, stream);
+
+    if (keep) {
+        for (int i = 0; i < 3; i++) kept[S_Q - NTENSORS + i] = qkv[i];
+        kept[S_QRAW - NTENSORS] = raw[0], kept[S_KRAW - NTENSORS] = raw[1], kept[S_Y - NTENSORS] = y, kept[S_LSE - NTENSORS] = lse;
+    }
+    return out;
+}
+
+// Gradients of the arguments that need one; t: the contiguous arguments (biases are not looked at) followed by what was kept.
+void layer_backward(const Tensor &grad, const Tensor *t, const LayerConfig &cfg, const std::array<bool, NGRADS> &needed, Tensor (&result)[NGRADS])
+{
+    auto need = [&](int i) { return needed[i]; };
+    auto give = [&](int i, const Tensor &g) { result[i] = g; };
+    const int64_t B = t[XQ].size(0), C = t[XQ].size(1), nh = cfg.num_heads, Ck = t[WQ].size(0), Cv = t[WV].size(0);
+    const int64_t Po = cfg.nlat_out * cfg.nlon_out, Pi = cfg.nlat_in * cfg.nlon_in;
+    const bool normed = t[NQ].defined();
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(t[XQ].device());
+    void *stream = current_stream(t[XQ].device());
+    const auto opt = t[XQ].options().dtype(cfg.compute);
+    const int comp = dtype_code(cfg.compute);
+    const Tensor g = grad.contiguous();
+    const auto srcs = sources(t[XK].defined(), t[XV].defined());
+    const int64_t ch[3] = {Ck, Ck, Cv};
+    bool through = false; // does anything ahead of the output projection need a gradient?
+    for (int i : {XQ, XK, XV, WQ, WK, WV, BQ, BK, BV, NQ, NK}) through |= need(i);
+
+    // transposed weights: of the output projection; of each input's projections, next to each other along the columns
+    Packer pk(comp);
+    int64_t p_ofs = 0, x_ofs[3] = {0, 0, 0};
+    if (through) {
+        p_ofs = pk.reserve(blocks64(Cv), pk.k16(Cv));
+        pk.add(t[WP], Tensor(), Cv, Cv, true, 1.0, p_ofs, -1, 0, 0, pk.k16(Cv));
+        for (size_t j = 0; j < srcs.size(); j++) {
+            if (!need(srcs[j].x)) continue;
+            int total = 0, at = 0;
+            for (int i = srcs[j].first; i < srcs[j].first + srcs[j].count; i++) total += pk.k16(ch[i]);
+            x_ofs[j] = pk.reserve(blocks64(C), total);
+            for (int i = srcs[j].first; i < srcs[j].first + srcs[j].count; i++) {
+                pk.add(t[WQ + i], Tensor(), C, ch[i], true, i == 0 && !normed ? cfg.scale : 1.0, x_ofs[j], -1, 0, at, total);
+                at += pk.k16(ch[i]);
+            }
+        }
+    }
+    const Tensor packed = through ? pk.run(t[XQ], stream) : Tensor();
+
+    Gradients gr{stream, {}, {}};
+    if (need(WP) || need(BP)) { // rows of the partial sums are y's channels, columns the gradient's
+        auto [part, sums, none, slices] = gr.partials(g, Cv, {{&t[S_Y], Cv}}, B, Po, comp, need(BP), false);
+        if (need(WP)) {
+            Tensor w = at::empty(t[WP].sizes(), t[WP].options());
+            gr.job(part.data_ptr<float>(), w, slices, Cv * Cv, Cv, Cv, 1, Cv, 1.0);
+            give(WP, w);
+        }
+        if (need(BP)) {
+            Tensor b = at::empty({Cv}, t[WP].options());
+            gr.job(sums.data_ptr<float>(), b, slices, Cv, 1, Cv, 0, 1, 1.0);
+            give(BP, b);
+        }
+    }
+    if (through) {
+        Tensor gy = at::empty(t[S_Y].sizes(), opt);
+        project(true, {{&g, Cv}}, {{&gy, Cv}}, B, Po, comp, at_byte(packed, p_ofs), nullptr, stream);
+        const auto [dk, dv, dq] = backward_impl(t[S_K], t[S_V], t[S_Q], gy, &t[S_Y], &t[S_LSE], t[QUAD], t[COL], t[ROW], nh, cfg.nlon_in, cfg.nlat_out,
+                                                cfg.nlon_out, t[PLAN], c10::OptionalArrayRef<int64_t>(cfg.plan_header));
+        const Tensor *d[3] = {&dq, &dk, &dv};
+        if (normed) { // the gradients of the normed q and k become those of the projected ones, in place
+            s2attn_norm n = {};
+            n.ntensors = 2, n.head_channels = (int)(Ck / nh), n.dtype = comp, n.gain_dtype = dtype_code(t[NQ].scalar_type()), n.eps = RMS_EPS;
+            n.blocks = 1024;
+            for (int i = 0; i < 2; i++) {
+                const Tensor part = at::empty({n.blocks * n.head_channels}, opt.dtype(at::kFloat));
+                gr.keep.push_back(part);
+                n.x[i] = t[S_QRAW + i].data_ptr(), n.y[i] = d[i]->data_ptr(), n.gain[i] = t[NQ + i].data_ptr(), n.mult[i] = i ? 1.f : (float)cfg.scale;
+                n.dgain[i] = part.data_ptr<float>(), n.rows[i] = B * (i ? Pi : Po) * nh;
+                if (need(NQ + i)) {
+                    Tensor w = at::empty(t[NQ + i].sizes(), t[NQ + i].options());
+                    gr.job(part.data_ptr<float>(), w, n.blocks, n.head_channels, 1, n.head_channels, 0, 1, n.mult[i]);
+                    give(NQ + i, w);
+                }
+            }
+            check_rc(s2attn_head_norm_backward(&n, stream), "s2attn_head_norm_backward");
+        }
+        for (size_t j = 0; j < srcs.size(); j++) {
+            const Source &s = srcs[j];
+            const int64_t points = s.x == XQ ? Po : Pi;
+            std::vector<Part> parts;
+            bool want_w = false, want_b = false;
+            int64_t cj = 0;
+            for (int i = s.first; i < s.first + s.count; i++) {
+                parts.push_back({d[i], ch[i]});
+                want_w |= need(WQ + i), want_b |= need(BQ + i), cj += ch[i];
+            }
+            if (need(s.x)) {
+                Tensor dx = at::empty_like(t[s.x]);
+                project(false, parts, {{&dx, C}}, B, points, comp, at_byte(packed, x_ofs[j]), nullptr, stream);
+                give(s.x, dx);
+            }
+            if (!want_w && !want_b) continue;
+            auto [part, none, sums, slices] = gr.partials(t[s.x], C, parts, B, points, comp, false, want_b);
+            int64_t at = 0;
+            for (int i = s.first; i < s.first + s.count; i++) {
+                const double scale = i == 0 && !normed ? cfg.scale : 1.0;
+                if (need(WQ + i)) {
+                    Tensor w = at::empty(t[WQ + i].sizes(), t[WQ + i].options());
+                    gr.job(part.data_ptr<float>() + at * C, w, slices, cj * C, ch[i], C, C, 1, scale);
+                    give(WQ + i, w);
+                }
+                if (need(BQ + i)) {
+                    Tensor b = at::empty({ch[i]}, t[WQ + i].options());
+                    gr.job(sums.data_ptr<float>() + at, b, slices, cj, 1, ch[i], 0, 1, scale);
+                    give(BQ + i, b);
+                }
+                at += ch[i];
+            }
+        }
+    }
+    gr.finish();
+}
+
+struct LayerFunction : public torch::autograd::Function<LayerFunction> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, at::TensorList given, const c10::intrusive_ptr<LayerState> &state, bool need_backward)
+    {
+        Tensor t[NTENSORS], kept[NKEPT];
+        for (int i = 0; i < NTENSORS; i++)
+            if (state->slot[i] >= 0) t[i] = given[state->slot[i]].contiguous();
+        Tensor out = layer_forward(t, state->cfg, need_backward, kept);
+        if (need_backward) {
+            torch::autograd::variable_list saved(NSAVED);
+            for (int i = 0; i < NTENSORS; i++)
+                if (i < BQ || i > BP) saved[i] = t[i];
+            for (int i = 0; i < NKEPT; i++) saved[NTENSORS + i] = kept[i];
+            ctx->save_for_backward(std::move(saved));
+            ctx->saved_data["state"] = c10::IValue::make_capsule(state);
+        }
+        return out;
+    }
+
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
+    {
+        const auto held = ctx->saved_data["state"].toCapsule();
+        const LayerState &state = *static_cast<const LayerState *>(held.get());
+        int ngiven = 0;
+        for (int s : state.slot) ngiven += s >= 0;
+        torch::autograd::variable_list result(ngiven + 2); // + the two arguments that are no tensors
+        if (!grads[0].defined()) return result;
+        if (c10::GradMode::is_enabled()) TORCH_WARN_ONCE("NeighborhoodAttentionS2: the gradients of a backward with create_graph=True are not differentiable themselves");
+        Tensor g[NGRADS];
+        std::array<bool, NGRADS> need;
+        for (int i = 0; i < NGRADS; i++) need[i] = state.slot[i] >= 0 && ctx->needs_input_grad(state.slot[i]);
+        const auto t = ctx->get_saved_variables();
+        layer_backward(grads[0], t.data(), state.cfg, need, g);
+        for (int i = 0; i < NGRADS; i++)
+            if (g[i].defined()) result[state.slot[i]] = g[i];
+        return result;
+    }
+};
+
+void check_layer(const Tensor (&t)[NTENSORS], const LayerConfig &cfg)
+{
+    for (const Tensor &x : t)
+        if (x.defined()) require_gpu(x, "a tensor of the layer", t[XQ].device());
+    const int64_t B = t[XQ].size(0), C = t[XQ].size(1), Ck = t[WQ].size(0), Cv = t[WV].size(0);
+    auto image = [&](const Tensor &x, int64_t h, int64_t w) {
+        return x.dim() == 4 && x.size(0) == B && x.size(1) == C && x.size(2) == h && x.size(3) == w && x.scalar_type() == t[XQ].scalar_type();
+    };
+    const Tensor &xk = t[XK].defined() ? t[XK] : t[XQ], &xv = t[XV].defined() ? t[XV] : xk;
+    TORCH_CHECK(B > 0 && C > 0 && image(t[XQ], cfg.nlat_out, cfg.nlon_out) && image(xk, cfg.nlat_in, cfg.nlon_in) && image(xv, cfg.nlat_in, cfg.nlon_in),
+                "query, key and value must be non-empty (B, channels, nlat, nlon) tensors of one dtype on the layer's grids");
+    TORCH_CHECK(t[WQ].numel() == Ck * C && t[WK].numel() == Ck * C && t[WK].size(0) == Ck && t[WV].numel() == Cv * C && t[WP].numel() == Cv * Cv && t[WP].size(0) == Cv,
+                "projection weights do not fit the channels");
+    TORCH_CHECK(cfg.num_heads > 0 && Ck % cfg.num_heads == 0 && Cv % cfg.num_heads == 0, "num_heads must divide the channels");
+    TORCH_CHECK(t[BQ].defined() == t[BK].defined() && t[BQ].defined() == t[BV].defined() && t[NQ].defined() == t[NK].defined(), "q, k and v have a bias, q and k a norm, all or none");
+    const int64_t want[] = {Ck, Ck, Cv, Cv, Ck / cfg.num_heads, Ck / cfg.num_heads};
+    for (int i = BQ; i <= NK; i++)
+        TORCH_CHECK(!t[i].defined() || (t[i].numel() == want[i - BQ] && t[i].scalar_type() == t[i <= BP ? i - (BQ - WQ) : (int)NQ].scalar_type()), "bias or norm weight of a wrong length or dtype");
+}
+
+#define LAYER_ARGS                                                                                                                                             \
+    const Tensor &query, const c10::optional<Tensor> &key, const c10::optional<Tensor> &value, const Tensor &wq, const Tensor &wk, const Tensor &wv,            \
+        const Tensor &wp, const c10::optional<Tensor> &bq, const c10::optional<Tensor> &bk, const c10::optional<Tensor> &bv, const c10::optional<Tensor> &bp,  \
+        const c10::optional<Tensor> &nq, const c10::optional<Tensor> &nk, double scale, const Tensor &quad_weights, const Tensor &col_idx,                     \
+        const Tensor &row_off, const Tensor &plan, c10::ArrayRef<int64_t> plan_header, int64_t num_heads, int64_t nlat_in, int64_t nlon_in,                    \
+        int64_t nlat_out, int64_t nlon_out, at::ScalarType compute
+#define LAYER_TENSORS                                                                                                                                          \
+    {query, key.value_or(Tensor()), value.value_or(Tensor()), wq, wk, wv, wp, bq.value_or(Tensor()), bk.value_or(Tensor()), bv.value_or(Tensor()),             \
+     bp.value_or(Tensor()), nq.value_or(Tensor()), nk.value_or(Tensor()), quad_weights, col_idx, row_off, plan}
+#define LAYER_CONFIG LayerConfig{num_heads, nlat_in, nlon_in, nlat_out, nlon_out, scale, compute, plan_header.vec()}
+
+// eager mode: one C++ autograd node
+Tensor module_attention(LAYER_ARGS)
+{
+    const Tensor t[NTENSORS] = LAYER_TENSORS;
+    auto state = c10::make_intrusive<LayerState>();
+    state->cfg = LAYER_CONFIG;
+    check_layer(t, state->cfg);
+    std::vector<Tensor> given;
+    given.reserve(NTENSORS);
+    bool need_backward = false;
+    for (int i = 0; i < NTENSORS; i++) {
+        state->slot[i] = t[i].defined() ? (int)given.size() : -1;
+        if (!t[i].defined()) continue;
+        need_backward |= t[i].requires_grad();
+        given.push_back(t[i]);
+    }
+    return LayerFunction::apply(at::TensorList(given), state, need_backward && c10::GradMode::is_enabled());
+}
+
+// the same two steps as operators without an autograd node of their own: what a compiled graph records (fake kernels and the autograd
+// rule in ops.py).  An absent tensor is returned as an empty one.
+std::vector<Tensor> layer_forward_op(LAYER_ARGS)
+{
+    const Tensor t[NTENSORS] = LAYER_TENSORS;
+    const LayerConfig cfg = LAYER_CONFIG;
+    check_layer(t, cfg);
+    Tensor kept[NKEPT];
+    std::vector<Tensor> r{layer_forward(t, cfg, true, kept)};
+    for (const Tensor &x : kept) r.push_back(x.defined() ? x : at::empty({0}, query.options().dtype(compute)));
+    return r;
+}
+
+std::vector<Tensor> layer_backward_op(const Tensor &grad, LAYER_ARGS, at::TensorList kept, std::array<bool, NGRADS> need)
+{
+    Tensor given[NTENSORS] = LAYER_TENSORS;
+    const LayerConfig cfg = LAYER_CONFIG;
+    check_layer(given, cfg);
+    TORCH_CHECK(kept.size() == NKEPT, "layer_backward takes the ", NKEPT, " tensors that layer_forward keeps");
+    std::vector<Tensor> t(NSAVED);
+    for (int i = 0; i < NTENSORS; i++)
+        if (given[i].defined()) t[i] = given[i].contiguous();
+    for (int i = 0; i < NKEPT; i++) t[NTENSORS + i] = kept[i];
+    Tensor g[NGRADS];
+    for (int i = 0; i < NGRADS; i++) need[i] = need[i] && given[i].defined();
+    layer_backward(grad, t.data(), cfg, need, g);
+    std::vector<Tensor> r;
+    for (const Tensor &x : g) r.push_back(x.defined() ? x : at::empty({0}, query.options()));
+    return r;
+}
+
 // ---- layout ---------------------------------------------------------------------------------------------------------------
 Tensor permute(const Tensor &x, bool to_nhwc)
 {
@@ -369,16 +804,28 @@ TORCH_LIBRARY(s2attn_kernels, m)
     m.def("backward_saved(Tensor kx, Tensor vx, Tensor qy, Tensor dy, Tensor y, Tensor lse, Tensor quad_weights, Tensor col_idx, Tensor row_off, int "
           "num_heads, int nlon_in, int nlat_out, int nlon_out, Tensor? plan=None, int[]? plan_header=None) -> (Tensor, Tensor, Tensor)",
           {at::Tag::pt2_compliant_tag});
+    // the layer: module_attention makes its autograd node inside, so it is a composite operator
+    const std::string layer =
+        "Tensor query, Tensor? key, Tensor? value, Tensor q_weights, Tensor k_weights, Tensor v_weights, Tensor proj_weights, Tensor? q_bias, Tensor? k_bias, "
+        "Tensor? v_bias, Tensor? proj_bias, Tensor? q_norm, Tensor? k_norm, float scale, Tensor quad_weights, Tensor col_idx, Tensor row_off, Tensor plan, "
+        "int[] plan_header, int num_heads, int nlat_in, int nlon_in, int nlat_out, int nlon_out, ScalarType compute";
+    m.def(("module_attention(" + layer + ") -> Tensor").c_str(), &module_attention);
+    m.def(("layer_forward(" + layer + ") -> Tensor[]").c_str(), {at::Tag::pt2_compliant_tag});
+    m.def(("layer_backward(Tensor grad, " + layer + ", Tensor[] kept, bool[13] need) -> Tensor[]").c_str(), {at::Tag::pt2_compliant_tag});
 }
 
 TORCH_LIBRARY_IMPL(s2attn_kernels, CUDA, m)
 {
     m.impl("forward_lse", &forward_lse);
     m.impl("backward_saved", &backward_saved);
+    m.impl("layer_forward", &layer_forward_op);
+    m.impl("layer_backward", &layer_backward_op);
 }
 
 TORCH_LIBRARY_IMPL(s2attn_kernels, CPU, m) // fails with the same message as above
 {
     m.impl("forward_lse", &forward_lse);
     m.impl("backward_saved", &backward_saved);
+    m.impl("layer_forward", &layer_forward_op);
+    m.impl("layer_backward", &layer_backward_op);
 }

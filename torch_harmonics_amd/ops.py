@@ -56,6 +56,11 @@ permute_to_nhwc = torch.ops.attention_kernels.permute_to_nhwc
 permute_to_nchw = torch.ops.attention_kernels.permute_to_nchw
 forward_lse = torch.ops.s2attn_kernels.forward_lse
 backward_saved = torch.ops.s2attn_kernels.backward_saved
+# the whole layer (projections, q/k norm, attention, output projection): one C++ autograd node in eager mode, and its forward and
+# backward as operators for compiled graphs (module_attention_traced, at the end of this file)
+module_attention = torch.ops.s2attn_kernels.module_attention.default
+layer_forward = torch.ops.s2attn_kernels.layer_forward.default
+layer_backward = torch.ops.s2attn_kernels.layer_backward.default
 
 
 @torch.library.register_fake("attention_kernels::forward")
@@ -259,6 +264,50 @@ def neighborhood_s2_attention(kw, vw, qw, quad_weights, col_idx, row_off, nh, nl
     """Differentiable attention on NHWC heads-packed tensors; what NeighborhoodAttentionS2.forward calls.  plan, plan_header:
     the psi's plan built ahead of time (the module builds it in its constructor), so that no call copies psi to the host."""
     return _neighborhood_s2_attention_saved(kw, vw, qw, quad_weights, col_idx, row_off, nh, nlon_in, nlat_out, nlon_out, plan, plan_header)[0]
+
+
+# The layer under torch.compile: the same kernels as module_attention, with fake kernels and an autograd rule the tracer can record.
+_LAYER_TENSORS = 13  # query, key, value, four weights, four biases, two norm gains: the arguments that may need a gradient
+
+
+@torch.library.register_fake("s2attn_kernels::layer_forward")
+def _(query, key, value, q_weights, k_weights, v_weights, proj_weights, q_bias, k_bias, v_bias, proj_bias, q_norm, k_norm, scale, quad_weights, col_idx,
+      row_off, plan, plan_header, num_heads, nlat_in, nlon_in, nlat_out, nlon_out, compute):  # fmt: skip
+    B, ck, cv = query.shape[0], q_weights.shape[0], v_weights.shape[0]
+    new = lambda *s: query.new_empty(s, dtype=compute)  # noqa: E731
+    q, k = new(B, nlat_out, nlon_out, ck), new(B, nlat_in, nlon_in, ck)
+    raw = (new(0), new(0)) if q_norm is None else (torch.empty_like(q), torch.empty_like(k))
+    lse = query.new_empty((B, num_heads, nlat_out, nlon_out), dtype=torch.float32)
+    return [new(B, cv, nlat_out, nlon_out), q, k, new(B, nlat_in, nlon_in, cv), *raw, new(B, nlat_out, nlon_out, cv), lse]
+
+
+@torch.library.register_fake("s2attn_kernels::layer_backward")
+def _(grad, *args):
+    tensors, kept, need = args[:_LAYER_TENSORS], args[-2], args[-1]  # noqa: F841
+    return [t.new_empty(t.shape) if n and t is not None else tensors[0].new_empty((0,)) for t, n in zip(tensors, need)]
+
+
+def _layer_setup_context(ctx, inputs, output):
+    ctx.save_for_backward(*inputs[:_LAYER_TENSORS], *inputs[14:18], *output[1:])
+    ctx.scale, ctx.rest = inputs[13], inputs[18:]
+    ctx.set_materialize_grads(False)
+
+
+def _layer_backward_rule(ctx, grads):
+    saved = ctx.saved_tensors
+    tensors, geometry, kept = saved[:_LAYER_TENSORS], saved[_LAYER_TENSORS : _LAYER_TENSORS + 4], saved[_LAYER_TENSORS + 4 :]
+    if grads[0] is None:
+        return (None,) * (_LAYER_TENSORS + 12)
+    need = [t is not None and bool(n) for t, n in zip(tensors, ctx.needs_input_grad)]
+    out = layer_backward(grads[0], *tensors, ctx.scale, *geometry, *ctx.rest, list(kept), need)
+    return (*[g if n else None for g, n in zip(out, need)], *(None,) * 12)
+
+
+torch.library.register_autograd("s2attn_kernels::layer_forward", _layer_backward_rule, setup_context=_layer_setup_context)
+
+
+def module_attention_traced(*args):
+    return layer_forward(*args)[0]
 
 
 # Autocast: k, v, q are brought to the active autocast dtype and the op re-entered with autocast off;
