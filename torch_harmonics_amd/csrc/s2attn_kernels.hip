@@ -28,6 +28,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
@@ -2276,6 +2277,7 @@ template <typename T> __global__ __launch_bounds__(64) void dkdv_mfma_kernel(con
 
 #include "s2attn_h16.hpp"
 #include "s2attn_m32.hpp"
+#include "s2attn_s16.hpp"
 
 // ---------------------------------------------------------------------------------
 // layout permutes: batched 2-D transpose [R, S] -> [S, R] through a 64x65 LDS tile
@@ -2312,6 +2314,7 @@ enum Which { FWD, DQ, DKDV };
 
 template <typename T, int D, bool PAD> int launch_h16(Which which, const Args &a0, hipStream_t stream);
 template <int D, int NS> int launch_m32(Which which, const Args &a0, hipStream_t stream);
+template <typename T, int D, bool PAD> int launch_s16(Which which, const Args &a0, hipStream_t stream);
 template <int D, int MODE, typename T> int launch_ring_m32(const Args &a0, hipStream_t stream);
 template <int D, bool WRITE, typename T> int launch_ring_pass2_m32(const Args &a0, hipStream_t stream);
 
@@ -2396,6 +2399,40 @@ template <int D, int NS> int launch_m32(Which which, const Args &a0, hipStream_t
     return S2ATTN_OK;
 }
 #endif
+#if S2_PART == 0 || S2_PART == 5
+// fp32 accuracy on bf16 matrix instructions, tiles of 16, 32, 48 or 64 channels
+template <typename T, int D, bool PAD> int launch_s16(Which which, const Args &a0, hipStream_t stream)
+{
+    Args a = a0;
+    a.row_first = 0;
+    void (*const kern)(const Args) = which == FWD ? fwd_s16_kernel<T, D, PAD> : which == DQ ? dq_s16_kernel<T, D, PAD> : dkdv_s16_kernel<T, D, PAD>;
+    const long nblocks = (which == DKDV ? (long)a.Hi * ((a.Wi + WQ - 1) / WQ) : (long)a.Ho * ((a.Wo + WQ - 1) / WQ)) * a.B * a.nh;
+    const int lds = s16_lds_bytes<T, D>(which == DKDV);
+    if (nblocks > 0x7fffffffL) return s2attn_fail(S2ATTN_E_UNSUPPORTED, "problem needs %ld workgroups, more than one grid holds", nblocks);
+    if (lds > 48 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return s2attn_fail(S2ATTN_E_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(64 * NW), lds, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return s2attn_fail(S2ATTN_E_LAUNCH, "kernel launch: %s", hipGetErrorString(e));
+    return S2ATTN_OK;
+}
+#endif
+#if S2_PART == 5
+template int launch_s16<float, 16, false>(Which, const Args &, hipStream_t);
+template int launch_s16<float, 32, false>(Which, const Args &, hipStream_t);
+template int launch_s16<float, 64, false>(Which, const Args &, hipStream_t);
+#define S2_S16_INSTANCES(T)                                            \
+    template int launch_s16<T, 16, true>(Which, const Args &, hipStream_t); \
+    template int launch_s16<T, 32, true>(Which, const Args &, hipStream_t); \
+    template int launch_s16<T, 48, true>(Which, const Args &, hipStream_t); \
+    template int launch_s16<T, 64, true>(Which, const Args &, hipStream_t);
+S2_S16_INSTANCES(float)
+S2_S16_INSTANCES(bf16_t)
+S2_S16_INSTANCES(f16_t)
+#undef S2_S16_INSTANCES
+#endif
 #if S2_PART == 0 || S2_PART == 3 || S2_PART == 4
 // one ring step (forward, or pass 1 of the backward) on the fp32 16-longitude kernels, tensors of storage type T: one wavefront per 16 local output longitudes
 template <int D, int MODE, typename T> int launch_ring_m32(const Args &a0, hipStream_t stream)
@@ -2443,8 +2480,6 @@ template int launch_ring_m32<128, 0, float>(const Args &, hipStream_t);
 template int launch_ring_m32<128, 1, float>(const Args &, hipStream_t);
 template int launch_ring_m32<128, 2, float>(const Args &, hipStream_t);
 template int launch_m32<16, 1>(Which, const Args &, hipStream_t);
-template int launch_m32<32, 1>(Which, const Args &, hipStream_t);
-template int launch_m32<64, 1>(Which, const Args &, hipStream_t);
 template int launch_m32<128, 1>(Which, const Args &, hipStream_t);
 template int launch_m32<128, 2>(Which, const Args &, hipStream_t);
 template int launch_m32<128, 3>(Which, const Args &, hipStream_t);
@@ -2665,9 +2700,9 @@ template <typename T> bool h16_ok(Which which, const Args &a)
     return true;
 }
 
-// Head widths: any multiple of 4 from 16 to 512, staged in a tile of 16, 32, 64 or 128 channels (zeros past the head), or in
-// two to four channel groups of 128 worked on by as many wavefronts.
-bool m32_width(int ck, int cv) { return ck == cv && ck % 4 == 0 && ck >= 16 && ck <= 512; }
+// Head widths above those of the split kernels: any multiples of 4 up to 512, q / k and v each its own, staged in a tile of 128
+// channels (zeros past the head), or in two to four channel groups of 128 worked on by as many wavefronts.
+bool m32_width(int ck, int cv) { return ck % 4 == 0 && cv % 4 == 0 && ck <= 512 && cv <= 512; }
 
 template <typename T> bool m32_ok(Which which, const Args &a)
 {
@@ -2677,6 +2712,45 @@ template <typename T> bool m32_ok(Which which, const Args &a)
     const void *ptrs[] = {a.k, a.v, a.q, a.dy, a.y, a.dk, a.dv, a.dq, a.ysaved};
     for (const void *p : ptrs)
         if (p && !aligned(p, 16)) return false;
+    return true;
+}
+
+// Head widths: any multiples of 4 up to 64, q / k and v each its own, in a tile of 16, 32, 48 or 64 channels.
+bool s16_width(int ck, int cv) { return ck % 4 == 0 && cv % 4 == 0 && ck <= 64 && cv <= 64; }
+
+template <typename T> bool s16_ok(Which which, const Args &a)
+{
+    if (!s16_width(a.dk_, a.dv_) || a.Wi < HK) return false;
+    if (which == DQ && !(a.ysaved && a.lse)) return false;
+    if (std::is_same<T, float>::value) return true;
+    const void *ptrs[] = {a.k, a.v, a.q, a.dy, a.y, a.dk, a.dv, a.dq, a.ysaved}; // rows are read as four 16-bit values
+    for (const void *p : ptrs)
+        if (p && !aligned(p, 8)) return false;
+    return true;
+}
+
+// fp32, where another family could take the problem too: are the split kernels the faster ones?
+bool s16_faster(Which which, const Args &a, int ndense)
+{
+    const int nv = which == DKDV ? a.Hi : a.Ho;
+    const bool long_runs = which == DKDV ? 2 * ndense >= nv : 3 * ndense >= nv; // on enough latitudes
+    const long nwg = (long)nv * ((a.Wi + WQ - 1) / WQ) * a.B * a.nh;
+    if (a.dk_ == 32 && a.dv_ == 32) {
+        // The hybrid kernels are the faster ones where most latitudes have short runs only (they take those
+        // neighbor by neighbor, these in steps of 32 positions) and the grid is large.  Measured on a 361 x 720 grid, share of long-run
+        // latitudes 0.24 / 0.29 / 0.39 / 0.48 / 0.60: forward 462 / 618 / 788 / 987 / 1176 us here, 405 / 607 / 850 / 1124 / 1420 there;
+        // dk/dv 717 / 974 / 1257 / 1565 / 1912 against 542 / 803 / 1141 / 1520 / 2001.  On small grids (91 x 180, four heads: 149
+        // against 249 us) a polar latitude's walk is what takes the time, and it is shorter here.
+        return long_runs || nwg < 4096;
+    }
+    if (std::max(a.dk_, a.dv_) <= 16) {
+        // The 16-longitude fp32 kernels read and stage a third of the bytes and have no barrier: the better ones on grids of few
+        // workgroups, where a step's latency is what counts (64 x 128, one head, four spacings: 21 / 25 / 32 us against 29 / 29 / 36), and
+        // in the forward and dk/dv over short runs (361 x 720, four heads, two spacings: 237 / 303 / 347 against 244 / 297 / 385;
+        // six: 728 / 857 / 1050 against 692 / 781 / 1082; 91 x 180, four: 40 / 50 / 64 against 41 / 45 / 54).
+        if (nwg < 1024) return false;
+        return which == DQ || long_runs || (which == DKDV && nwg < 4096);
+    }
     return true;
 }
 
@@ -2690,12 +2764,22 @@ template <typename T> int launch_t(Which which, const Args &a, bool vec, int nde
 {
     const int nrows = which == DKDV ? a.Hi : a.Ho;
     int first = 0;
-    if (a.unpacked) { // column blocks of a wider buffer: only the hybrid kernels address every tensor by its own point stride
-        if (!dense_ok(which, a, vec))
-            return s2attn_fail(S2ATTN_E_UNSUPPORTED, "tensors with a point stride need the hybrid kernels: ck = cv = 32, 16-byte aligned, at least 64 longitudes%s",
-                               which == DQ ? ", backward from saved statistics" : "");
-        return launch_dense<T>(which, a, stream);
+    // column blocks of a wider buffer: only the hybrid and the split kernels address every tensor by its own point stride, and
+    // callers rely on the former's domain
+    if (a.unpacked && !dense_ok(which, a, vec))
+        return s2attn_fail(S2ATTN_E_UNSUPPORTED, "tensors with a point stride need the hybrid kernels: ck = cv = 32, 16-byte aligned, at least 64 longitudes%s",
+                           which == DQ ? ", backward from saved statistics" : "");
+    const int d = std::max(a.dk_, a.dv_);
+    if constexpr (std::is_same<T, float>::value) {
+        if (s16_ok<T>(which, a) && (s16_faster(which, a, ndense) || !(dense_ok(which, a, vec) || (d <= 16 && m32_ok<T>(which, a))))) {
+            const bool exact = a.dk_ == a.dv_;
+            if (d <= 16) return exact && d == 16 ? launch_s16<T, 16, false>(which, a, stream) : launch_s16<T, 16, true>(which, a, stream);
+            if (d <= 32) return exact && d == 32 ? launch_s16<T, 32, false>(which, a, stream) : launch_s16<T, 32, true>(which, a, stream);
+            if (d <= 48) return launch_s16<T, 48, true>(which, a, stream);
+            return exact && d == 64 ? launch_s16<T, 64, false>(which, a, stream) : launch_s16<T, 64, true>(which, a, stream);
+        }
     }
+    if (a.unpacked) return launch_dense<T>(which, a, stream);
     if (h16_ok<T>(which, a)) {
         if (a.dk_ == 32) return launch_h16<T, 32, false>(which, a, stream);
         if (a.dk_ == 64) return launch_h16<T, 64, false>(which, a, stream);
@@ -2705,19 +2789,23 @@ template <typename T> int launch_t(Which which, const Args &a, bool vec, int nde
         if (a.dk_ < 128) return launch_h16<T, 128, true>(which, a, stream);
         return launch_h16<T, 256, true>(which, a, stream);
     }
+    if constexpr (!std::is_same<T, float>::value) {
+        if (s16_ok<T>(which, a)) {
+            if (d <= 16) return launch_s16<T, 16, true>(which, a, stream);
+            if (d <= 32) return launch_s16<T, 32, true>(which, a, stream);
+            return d <= 48 ? launch_s16<T, 48, true>(which, a, stream) : launch_s16<T, 64, true>(which, a, stream);
+        }
+    }
     if (dense_ok(which, a, vec)) {
         // head dim 32 on at least 64 columns: the hybrid kernels handle short runs themselves (vector path inside), so
         // they take every latitude; measured ahead of the 16-longitude family there (cfg3 13.5 against 16.4 ms)
-        (void)ndense;
         return launch_dense<T>(which, a, stream);
     }
     if (m32_ok<T>(which, a)) {
-        if (a.dk_ <= 16) return launch_m32<16, 1>(which, a, stream);
-        if (a.dk_ <= 32) return launch_m32<32, 1>(which, a, stream);
-        if (a.dk_ <= 64) return launch_m32<64, 1>(which, a, stream);
-        if (a.dk_ <= 128) return launch_m32<128, 1>(which, a, stream);
-        if (a.dk_ <= 256) return launch_m32<128, 2>(which, a, stream);
-        return a.dk_ <= 384 ? launch_m32<128, 3>(which, a, stream) : launch_m32<128, 4>(which, a, stream);
+        if (d <= 16) return launch_m32<16, 1>(which, a, stream);
+        if (d <= 128) return launch_m32<128, 1>(which, a, stream);
+        if (d <= 256) return launch_m32<128, 2>(which, a, stream);
+        return d <= 384 ? launch_m32<128, 3>(which, a, stream) : launch_m32<128, 4>(which, a, stream);
     }
     return vec ? launch_p<T, true>(which, a, first, nrows - first, stream) : launch_p<T, false>(which, a, first, nrows - first, stream);
 }
@@ -2841,7 +2929,7 @@ int ring_plan_args(Args &a, const void *k, const void *v, const void *q, const v
                            h[S2ATTN_PH_NLAT_IN], h[S2ATTN_PH_NLON_IN], h[S2ATTN_PH_NLAT_OUT], h[S2ATTN_PH_NLON_OUT], g.qps > 1 ? "the chunk's latitudes" : "all input latitudes",
                            g.nlon_in, g.nlat_out, wout);
     if (g.dtype != S2ATTN_F32 && g.dtype != S2ATTN_BF16 && g.dtype != S2ATTN_F16) return s2attn_fail(S2ATTN_E_INVALID, "unknown dtype code %d", g.dtype);
-    if (!m32_width(g.ck, g.cv) || g.ck > 128 || W < HK)
+    if (g.ck != g.cv || g.ck % 4 != 0 || g.ck < 16 || g.ck > 128 || W < HK)
         return s2attn_fail(S2ATTN_E_UNSUPPORTED, "the band-staged ring steps take tensors with ck = cv a multiple of 4 from 16 to 128 on at least %d longitudes", HK);
     const void *ptrs[] = {k, v, q, dy};
     const int need = g.dtype == S2ATTN_F32 ? 16 : 8; // four channels are loaded at a time
@@ -3006,9 +3094,9 @@ namespace {
 bool h16_shape(const s2attn_shape *sh)
 {
     const int w = sh->nlon_out < sh->nlon_in ? sh->nlon_out : sh->nlon_in; // columns of a virtual latitude
-    if (sh->ck != sh->cv || w < HK) return false;
-    if (sh->dtype == S2ATTN_F32) return m32_width(sh->ck, sh->cv); // the fp32 16-longitude family and the hybrid kernels work the same way
-    return h16_width(sh->ck, sh->cv);
+    if (w < HK) return false;
+    if (sh->dtype == S2ATTN_F32) return s16_width(sh->ck, sh->cv) || m32_width(sh->ck, sh->cv); // the fp32 16-longitude family and the hybrid kernels work the same way
+    return h16_width(sh->ck, sh->cv) || s16_width(sh->ck, sh->cv);
 }
 int64_t stat_points(const s2attn_shape *sh) { return (int64_t)sh->batch * sh->num_heads * sh->nlat_out * sh->nlon_out; }
 int64_t round16(int64_t n) { return (n + 15) / 16 * 16; }

@@ -3,7 +3,7 @@
 // HQ = 16 consecutive longitudes of one latitude for one (batch, head) and walks every run of that latitude in steps of
 // HK = 32 band positions; lane l = (c = l % 16, qd = l / 16); scores are produced transposed, S^T[position][column].
 //
-// Shape domain: ck == cv = dr, a multiple of 4 with dr <= D (the tile is D channels wide; channels from dr on are staged
+// Shape domain: ck and cv multiples of 4, both at most D (the tile is D channels wide; channels past a head's are staged
 // as zeros and never stored), at least 32 columns per virtual latitude, 16-byte aligned rows.
 //
 // Facts about the instruction:  A operand: the lane supplies A[i = c][k = qd];  B operand: B[k = qd][j = c];
@@ -35,9 +35,9 @@
     const int b = bh / a.nh, h = bh % a.nh;                                   \
     const int w0 = wt * HQ;                                                   \
     const int nvalid = min(HQ, (W_TILED)-w0);                                 \
-    const int drt = a.dk_;                 /* real head width */              \
     const int cbase = wv * D;              /* first channel of this wavefront's group */ \
-    const int dr = min(D, drt - cbase);    /* real channels in the group */
+    const int nk = min(D, a.dk_ - cbase), nv = min(D, a.dv_ - cbase); /* channels of q / k and of v in the group (may be none) */ \
+    const unsigned ldbk_ = a.nh * a.dk_ * 4, ldbv_ = a.nh * a.dv_ * 4; /* bytes between two grid points */
 
 extern __shared__ float4 m32_smem[];
 
@@ -184,14 +184,13 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kern
     char *Ks = lds + wv * m32_wave_bytes<D, NS>(false), *Vs = Ks + HK * PITCH;
     float *xs = reinterpret_cast<float *>(lds + NS * m32_wave_bytes<D, NS>(false));
     const int ho = a.gorder[a.row_first + rowsel];
-    const unsigned ldb = a.nh * drt * 4; // bytes between two grid points
-    const char *kx = static_cast<const char *>(a.k) + ((size_t)b * a.Hi * a.Wi * a.nh + h) * (drt * 4) + cbase * 4;
-    const char *vx = static_cast<const char *>(a.v) + ((size_t)b * a.Hi * a.Wi * a.nh + h) * (drt * 4) + cbase * 4;
+    const char *kx = static_cast<const char *>(a.k) + ((size_t)b * a.Hi * a.Wi * a.nh + h) * (a.dk_ * 4) + cbase * 4;
+    const char *vx = static_cast<const char *>(a.v) + ((size_t)b * a.Hi * a.Wi * a.nh + h) * (a.dv_ * 4) + cbase * 4;
     const bool mine = c < nvalid;
     const size_t pt = (size_t)query_point(a, b, ho, ho / a.qps) + (size_t)(w0 + (mine ? c : 0)) * a.qps;
 
     float qop[D / 4];
-    m32_load_quarter<D>(qop, static_cast<const char *>(a.q) + pt * ldb + (size_t)h * (drt * 4) + cbase * 4, qd, dr);
+    m32_load_quarter<D>(qop, static_cast<const char *>(a.q) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4, qd, nk);
     f4v acc[NCB]; // Y^T: register v of block cb is channel 16 cb + 4 qd + v of column c
 #pragma unroll
     for (int cb = 0; cb < NCB; cb++) acc[cb] = f4v{0.f, 0.f, 0.f, 0.f};
@@ -202,16 +201,17 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kern
     int pos = 0;
     Run run = {0, 0, 0, 0};
     Tile kt, vt;
-    const unsigned ldbk = ldb * a.kps; // bytes between two columns of a virtual input latitude
-    const unsigned lane_off = (unsigned)(lane / Tile::CPR) * ldbk + 16u * (lane % Tile::CPR);
-    const bool piece_ok = 4 * (lane % Tile::CPR) < dr; // this lane's 16-byte piece of a staged row exists
+    const unsigned ldbk = ldbk_ * a.kps, ldbv = ldbv_ * a.kps; // bytes between two columns of a virtual input latitude
+    const unsigned lane_k = (unsigned)(lane / Tile::CPR) * ldbk + 16u * (lane % Tile::CPR), lane_v = (unsigned)(lane / Tile::CPR) * ldbv + 16u * (lane % Tile::CPR);
+    const bool k_ok = 4 * (lane % Tile::CPR) < nk, v_ok = 4 * (lane % Tile::CPR) < nv; // this lane's 16-byte piece of a staged row exists
     auto fetch = [&](const Run &rn, int p) {
         const int c0 = (rn.ws + w0 + p) % a.Wi;
         unsigned off[Tile::NIT];
-        Tile::offsets(off, lane_off, lane, c0, a.Wi, ldbk);
-        const size_t lat_off = (size_t)key_row(a, rn.lat, rn.pad) * ldb;
-        kt.fetch_if(kx + lat_off, off, piece_ok);
-        vt.fetch_if(vx + lat_off, off, piece_ok);
+        const size_t row = (size_t)key_row(a, rn.lat, rn.pad);
+        Tile::offsets(off, lane_k, lane, c0, a.Wi, ldbk);
+        kt.fetch_if(kx + row * ldbk_, off, k_ok);
+        if (ldbv != ldbk) Tile::offsets(off, lane_v, lane, c0, a.Wi, ldbv);
+        vt.fetch_if(vx + row * ldbv_, off, v_ok);
     };
     if (ri < rend) {
         run = a.gruns[ri];
@@ -294,10 +294,10 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kern
     if (mine) {
         if (a.lse && qd == 0 && wv == 0) a.lse[((size_t)bh * a.Ho + ho) * a.Wo + w0 + c] = m + fast_log2(S);
         const float inv = 1.0f / S;
-        char *y = static_cast<char *>(a.y) + pt * ldb + (size_t)h * (drt * 4) + cbase * 4 + 16 * qd;
+        char *y = static_cast<char *>(a.y) + pt * ldbv_ + (size_t)h * (a.dv_ * 4) + cbase * 4 + 16 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++)
-            if (16 * cb + 4 * qd < dr)
+            if (16 * cb + 4 * qd < nv)
                 *reinterpret_cast<float4 *>(y + 64 * cb) = make_float4(acc[cb][0] * inv, acc[cb][1] * inv, acc[cb][2] * inv, acc[cb][3] * inv);
     }
 }
@@ -313,9 +313,8 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dq_m32_kerne
     char *Ks = lds + wv * m32_wave_bytes<D, NS>(false), *Vs = Ks + HK * PITCH;
     float *xs = reinterpret_cast<float *>(lds + NS * m32_wave_bytes<D, NS>(false));
     const int ho = a.gorder[a.row_first + rowsel];
-    const unsigned ldb = a.nh * drt * 4;
-    const char *kx = static_cast<const char *>(a.k) + ((size_t)b * a.Hi * a.Wi * a.nh + h) * (drt * 4) + cbase * 4;
-    const char *vx = static_cast<const char *>(a.v) + ((size_t)b * a.Hi * a.Wi * a.nh + h) * (drt * 4) + cbase * 4;
+    const char *kx = static_cast<const char *>(a.k) + ((size_t)b * a.Hi * a.Wi * a.nh + h) * (a.dk_ * 4) + cbase * 4;
+    const char *vx = static_cast<const char *>(a.v) + ((size_t)b * a.Hi * a.Wi * a.nh + h) * (a.dv_ * 4) + cbase * 4;
     const bool mine = c < nvalid;
     const size_t pt = (size_t)query_point(a, b, ho, ho / a.qps) + (size_t)(w0 + (mine ? c : 0)) * a.qps;
     const size_t sidx = ((size_t)bh * a.Ho + ho) * a.Wo + w0 + (mine ? c : 0);
@@ -323,11 +322,11 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dq_m32_kerne
     float qop[D / 4], gop[D / 4];
     float I = 0.f;
     {
-        const size_t off = pt * ldb + (size_t)h * (drt * 4) + cbase * 4;
-        m32_load_quarter<D>(qop, static_cast<const char *>(a.q) + off, qd, dr);
-        m32_load_quarter<D>(gop, static_cast<const char *>(a.dy) + off, qd, dr);
+        const size_t off = pt * ldbv_ + (size_t)h * (a.dv_ * 4) + cbase * 4;
+        m32_load_quarter<D>(qop, static_cast<const char *>(a.q) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4, qd, nk);
+        m32_load_quarter<D>(gop, static_cast<const char *>(a.dy) + off, qd, nv);
         float yq[D / 4];
-        m32_load_quarter<D>(yq, static_cast<const char *>(a.ysaved) + off, qd, dr);
+        m32_load_quarter<D>(yq, static_cast<const char *>(a.ysaved) + off, qd, nv);
 #pragma unroll
         for (int i = 0; i < D / 4; i++) I = fmaf(gop[i], yq[i], I);
     }
@@ -352,16 +351,17 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dq_m32_kerne
     int pos = 0;
     Run run = {0, 0, 0, 0};
     Tile kt, vt;
-    const unsigned ldbk = ldb * a.kps;
-    const unsigned lane_off = (unsigned)(lane / Tile::CPR) * ldbk + 16u * (lane % Tile::CPR);
-    const bool piece_ok = 4 * (lane % Tile::CPR) < dr; // this lane's 16-byte piece of a staged row exists
+    const unsigned ldbk = ldbk_ * a.kps, ldbv = ldbv_ * a.kps;
+    const unsigned lane_k = (unsigned)(lane / Tile::CPR) * ldbk + 16u * (lane % Tile::CPR), lane_v = (unsigned)(lane / Tile::CPR) * ldbv + 16u * (lane % Tile::CPR);
+    const bool k_ok = 4 * (lane % Tile::CPR) < nk, v_ok = 4 * (lane % Tile::CPR) < nv; // this lane's 16-byte piece of a staged row exists
     auto fetch = [&](const Run &rn, int p) {
         const int c0 = (rn.ws + w0 + p) % a.Wi;
         unsigned off[Tile::NIT];
-        Tile::offsets(off, lane_off, lane, c0, a.Wi, ldbk);
-        const size_t lat_off = (size_t)key_row(a, rn.lat, rn.pad) * ldb;
-        kt.fetch_if(kx + lat_off, off, piece_ok);
-        vt.fetch_if(vx + lat_off, off, piece_ok);
+        const size_t row = (size_t)key_row(a, rn.lat, rn.pad);
+        Tile::offsets(off, lane_k, lane, c0, a.Wi, ldbk);
+        kt.fetch_if(kx + row * ldbk_, off, k_ok);
+        if (ldbv != ldbk) Tile::offsets(off, lane_v, lane, c0, a.Wi, ldbv);
+        vt.fetch_if(vx + row * ldbv_, off, v_ok);
     };
     if (ri < rend) {
         run = a.gruns[ri];
@@ -427,10 +427,10 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dq_m32_kerne
     // which the compiler only uses while nothing in the kernel can have written memory, into vector loads with waits)
     if (mine && qd == 0 && wv == 0) a.stats[sidx] = make_float2(lse, I);
     if (mine) {
-        char *dq = static_cast<char *>(a.dq) + pt * ldb + (size_t)h * (drt * 4) + cbase * 4 + 16 * qd;
+        char *dq = static_cast<char *>(a.dq) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4 + 16 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++)
-            if (16 * cb + 4 * qd < dr) *reinterpret_cast<float4 *>(dq + 64 * cb) = make_float4(acc[cb][0], acc[cb][1], acc[cb][2], acc[cb][3]);
+            if (16 * cb + 4 * qd < nk) *reinterpret_cast<float4 *>(dq + 64 * cb) = make_float4(acc[cb][0], acc[cb][1], acc[cb][2], acc[cb][3]);
     }
 }
 
@@ -448,18 +448,16 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dkdv_m32_ker
     float *Ls = reinterpret_cast<float *>(Gs + HK * PITCH), *Is = Ls + HK;
     float *xs = reinterpret_cast<float *>(lds + NS * m32_wave_bytes<D, NS>(true));
     const int hi = a.sorder[a.row_first + rowsel];
-    const unsigned ldb = a.nh * drt * 4;
-    const char *qy = static_cast<const char *>(a.q) + ((size_t)b * a.Ho * a.Wo * a.nh + h) * (drt * 4) + cbase * 4;
-    const char *gy = static_cast<const char *>(a.dy) + ((size_t)b * a.Ho * a.Wo * a.nh + h) * (drt * 4) + cbase * 4;
+    const char *qy = static_cast<const char *>(a.q) + ((size_t)b * a.Ho * a.Wo * a.nh + h) * (a.dk_ * 4) + cbase * 4;
+    const char *gy = static_cast<const char *>(a.dy) + ((size_t)b * a.Ho * a.Wo * a.nh + h) * (a.dv_ * 4) + cbase * 4;
     const float2 *stats = a.stats + (size_t)bh * a.Ho * a.Wo;
     const bool mine = c < nvalid;
     const size_t pt = (size_t)key_point(a, b, hi, hi / a.kps) + (size_t)(w0 + (mine ? c : 0)) * a.kps;
 
     float kop[D / 4], vop[D / 4]; // this lane's quarter of key c
     {
-        const size_t off = pt * ldb + (size_t)h * (drt * 4) + cbase * 4;
-        m32_load_quarter<D>(kop, static_cast<const char *>(a.k) + off, qd, dr);
-        m32_load_quarter<D>(vop, static_cast<const char *>(a.v) + off, qd, dr);
+        m32_load_quarter<D>(kop, static_cast<const char *>(a.k) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4, qd, nk);
+        m32_load_quarter<D>(vop, static_cast<const char *>(a.v) + pt * ldbv_ + (size_t)h * (a.dv_ * 4) + cbase * 4, qd, nv);
     }
     f4v dkt[NCB], dvt[NCB];
 #pragma unroll
@@ -475,17 +473,18 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dkdv_m32_ker
     Run run = {0, 0, 0, 0};
     Tile qt, gt;
     float2 st = make_float2(0.f, 0.f);
-    const unsigned ldbq = ldb * a.qps; // bytes between two columns of a virtual output latitude
-    const unsigned lane_off = (unsigned)(lane / Tile::CPR) * ldbq + 16u * (lane % Tile::CPR);
-    const bool piece_ok = 4 * (lane % Tile::CPR) < dr; // this lane's 16-byte piece of a staged row exists
+    const unsigned ldbq = ldbk_ * a.qps, ldbg = ldbv_ * a.qps; // bytes between two columns of a virtual output latitude
+    const unsigned lane_q = (unsigned)(lane / Tile::CPR) * ldbq + 16u * (lane % Tile::CPR), lane_g = (unsigned)(lane / Tile::CPR) * ldbg + 16u * (lane % Tile::CPR);
+    const bool q_ok = 4 * (lane % Tile::CPR) < nk, g_ok = 4 * (lane % Tile::CPR) < nv; // this lane's 16-byte piece of a staged row exists
     auto fetch = [&](const Run &rn, int p) {
         int c0 = (w0 - rn.ws - rn.len + 1 + p) % a.Wo; // longitude of staged row 0
         c0 += (c0 < 0) ? a.Wo : 0;
         unsigned off[Tile::NIT];
-        Tile::offsets(off, lane_off, lane, c0, a.Wo, ldbq);
-        const size_t lat_off = (size_t)query_row(a, rn.lat, rn.pad) * ldb;
-        qt.fetch_if(qy + lat_off, off, piece_ok);
-        gt.fetch_if(gy + lat_off, off, piece_ok);
+        const size_t row = (size_t)query_row(a, rn.lat, rn.pad);
+        Tile::offsets(off, lane_q, lane, c0, a.Wo, ldbq);
+        qt.fetch_if(qy + row * ldbk_, off, q_ok);
+        if (ldbg != ldbq) Tile::offsets(off, lane_g, lane, c0, a.Wo, ldbg);
+        gt.fetch_if(gy + row * ldbv_, off, g_ok);
         int col = c0 + lane; // lanes 0..31 fetch the statistics of the staged rows
         col -= (col >= a.Wo) ? a.Wo : 0;
         if (lane < HK) st = stats[(size_t)rn.lat * a.Wo + col];
@@ -551,14 +550,12 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dkdv_m32_ker
     }
 
     if (mine) {
-        const size_t off = pt * ldb + (size_t)h * (drt * 4) + cbase * 4 + 16 * qd;
-        char *dk = static_cast<char *>(a.dk) + off, *dv = static_cast<char *>(a.dv) + off;
+        char *dk = static_cast<char *>(a.dk) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4 + 16 * qd;
+        char *dv = static_cast<char *>(a.dv) + pt * ldbv_ + (size_t)h * (a.dv_ * 4) + cbase * 4 + 16 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++) {
-            if (16 * cb + 4 * qd < dr) {
-                *reinterpret_cast<float4 *>(dk + 64 * cb) = make_float4(dkt[cb][0], dkt[cb][1], dkt[cb][2], dkt[cb][3]);
-                *reinterpret_cast<float4 *>(dv + 64 * cb) = make_float4(dvt[cb][0], dvt[cb][1], dvt[cb][2], dvt[cb][3]);
-            }
+            if (16 * cb + 4 * qd < nk) *reinterpret_cast<float4 *>(dk + 64 * cb) = make_float4(dkt[cb][0], dkt[cb][1], dkt[cb][2], dkt[cb][3]);
+            if (16 * cb + 4 * qd < nv) *reinterpret_cast<float4 *>(dv + 64 * cb) = make_float4(dvt[cb][0], dvt[cb][1], dvt[cb][2], dvt[cb][3]);
         }
     }
 }
@@ -647,6 +644,8 @@ template <int D, int MODE, typename T> __global__ __launch_bounds__(64, (D <= 32
     typedef FTile<D> Tile;
     constexpr int PITCH = Tile::PITCH, NCB = D / 16;
     S2_M32_IDS(a.Wo, a.Ho)
+    const int drt = a.dk_, dr = nk; // q, k and v have one width here
+    (void)nv, (void)ldbk_, (void)ldbv_;
     (void)h; // heads are folded into the batch
     (void)nvalid;
     char *lds = m32_lds<m32_lds_bytes<D, 1>(false), 1>();
