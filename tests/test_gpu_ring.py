@@ -68,6 +68,23 @@ def test_band_staged_ring_steps_take_16_bit_storage(case, dtype, d, monkeypatch)
     assert taken and all(taken)
 
 
+# windows and chunks that cross the 64-column tiles of the split-product ring steps; a circle that is local as a whole, in one tile and
+# narrower than one, with every point seeing every point (bands longer than the circle)
+SPLIT_CASES = [
+    ((7, 150), (7, 150), "equiangular", "equiangular", 0.45, (0, 7, 11, 117), [0, 115, 150]),
+    ((6, 64), (6, 64), "equiangular", "equiangular", 7.0, (0, 6, 0, 64), [0, 64]),
+    ((6, 34), (6, 34), "legendre-gauss", "legendre-gauss", 7.0, (0, 6, 0, 34), [0, 33, 34]),
+]
+SPLIT_WIDTHS = [(torch.float32, 20), (torch.float32, 32), (torch.float32, 48), (torch.bfloat16, 20), (torch.bfloat16, 64), (torch.float16, 32), (torch.float16, 36)]
+
+
+@pytest.mark.parametrize("dtype,d", SPLIT_WIDTHS, ids=lambda x: str(x).replace("torch.", ""))
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=lambda c: f"{c[0][0]}x{c[0][1]}_win{c[5]}")
+def test_split_product_ring_steps_at_the_edges_of_their_tiles(case, dtype, d, monkeypatch):
+    """Tolerances as everywhere else in this file: 1e-5 for the state (32-bit sums; the split adds at most 2^-23 per product)."""
+    _gather_direction(case, dtype, d, d, monkeypatch)
+
+
 def _gather_direction(case, dtype, ck, cv, monkeypatch):
     from torch_harmonics_amd import ops
 

@@ -36,10 +36,11 @@
 
 #include "s2attn_internal.h"
 
-// This file is compiled four times (see the Makefile), so that the groups of kernel instantiations build side by
+// This file is compiled six times (see the Makefile), so that the groups of kernel instantiations build side by
 // side: S2_PART 1 = everything but the launchers of the 16-longitude matrix-core families, 2 = the 16-bit family
-// (s2attn_h16.hpp), 3 = the fp32 family (s2attn_m32.hpp), 4 = its ring-step kernels for 16-bit storage.  S2_PART 0 (the
-// default) is the whole library in one unit.
+// (s2attn_h16.hpp), 3 = the fp32 family (s2attn_m32.hpp), 4 = its ring-step kernels for 16-bit storage, 5 = the split-product family
+// (s2attn_s16.hpp), 6 = its ring steps
+// (s2attn_s16_ring.hpp).  S2_PART 0 (the default) is the whole library in one unit.
 #ifndef S2_PART
 #define S2_PART 0
 #endif
@@ -2278,6 +2279,7 @@ template <typename T> __global__ __launch_bounds__(64) void dkdv_mfma_kernel(con
 #include "s2attn_h16.hpp"
 #include "s2attn_m32.hpp"
 #include "s2attn_s16.hpp"
+#include "s2attn_s16_ring.hpp"
 
 // ---------------------------------------------------------------------------------
 // layout permutes: batched 2-D transpose [R, S] -> [S, R] through a 64x65 LDS tile
@@ -2315,6 +2317,7 @@ enum Which { FWD, DQ, DKDV };
 template <typename T, int D, bool PAD> int launch_h16(Which which, const Args &a0, hipStream_t stream);
 template <int D, int NS> int launch_m32(Which which, const Args &a0, hipStream_t stream);
 template <typename T, int D, bool PAD> int launch_s16(Which which, const Args &a0, hipStream_t stream);
+template <typename T, int D, bool PAD, int MODE> int launch_ring_s16(const Args &a0, hipStream_t stream);
 template <int D, int MODE, typename T> int launch_ring_m32(const Args &a0, hipStream_t stream);
 template <int D, bool WRITE, typename T> int launch_ring_pass2_m32(const Args &a0, hipStream_t stream);
 
@@ -2433,6 +2436,46 @@ S2_S16_INSTANCES(bf16_t)
 S2_S16_INSTANCES(f16_t)
 #undef S2_S16_INSTANCES
 #endif
+#if S2_PART == 0 || S2_PART == 6
+// ring steps on split products: MODE 0 .. 2 as ring_s16_kernel, 3: pass 2, added to, 4: pass 2, written
+template <typename T, int D, bool PAD, int MODE> int launch_ring_s16(const Args &a0, hipStream_t stream)
+{
+    Args a = a0;
+    a.row_first = 0;
+    void (*kern)(const Args) = nullptr;
+    if constexpr (MODE < 3)
+        kern = ring_s16_kernel<T, D, PAD, MODE>;
+    else
+        kern = ring_pass2_s16_kernel<T, D, PAD, MODE == 4>;
+    const long nblocks = (MODE < 3 ? (long)a.Ho * ((a.Wo + WQ - 1) / WQ) : (long)a.Hi * ring_pass2_tiles(a.r_nkx, a.kps)) * a.B;
+    const int lds = s16_lds_bytes<T, D>(MODE >= 3);
+    if (nblocks > 0x7fffffffL) return s2attn_fail(S2ATTN_E_UNSUPPORTED, "problem needs %ld workgroups, more than one grid holds", nblocks);
+    if (lds > 48 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return s2attn_fail(S2ATTN_E_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(64 * NW), lds, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return s2attn_fail(S2ATTN_E_LAUNCH, "kernel launch: %s", hipGetErrorString(e));
+    return S2ATTN_OK;
+}
+#endif
+#if S2_PART == 6
+#define S2_RING_MODES(T, D)                                                    \
+    template int launch_ring_s16<T, D, true, 0>(const Args &, hipStream_t);    \
+    template int launch_ring_s16<T, D, true, 1>(const Args &, hipStream_t);    \
+    template int launch_ring_s16<T, D, true, 2>(const Args &, hipStream_t);    \
+    template int launch_ring_s16<T, D, true, 3>(const Args &, hipStream_t);    \
+    template int launch_ring_s16<T, D, true, 4>(const Args &, hipStream_t);
+#define S2_RING_INSTANCES(T) S2_RING_MODES(T, 32) S2_RING_MODES(T, 48) S2_RING_MODES(T, 64)
+S2_RING_INSTANCES(bf16_t)
+S2_RING_INSTANCES(f16_t)
+S2_RING_MODES(float, 48)
+template int launch_ring_s16<float, 32, true, 3>(const Args &, hipStream_t);
+template int launch_ring_s16<float, 32, false, 3>(const Args &, hipStream_t);
+#undef S2_RING_INSTANCES
+#undef S2_RING_MODES
+#endif
 #if S2_PART == 0 || S2_PART == 3 || S2_PART == 4
 // one ring step (forward, or pass 1 of the backward) on the fp32 16-longitude kernels, tensors of storage type T: one wavefront per 16 local output longitudes
 template <int D, int MODE, typename T> int launch_ring_m32(const Args &a0, hipStream_t stream)
@@ -2491,21 +2534,6 @@ template int launch_ring_pass2_m32<16, true, bf16_t>(const Args &, hipStream_t);
 template int launch_ring_m32<16, 0, bf16_t>(const Args &, hipStream_t);
 template int launch_ring_m32<16, 1, bf16_t>(const Args &, hipStream_t);
 template int launch_ring_m32<16, 2, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_pass2_m32<32, false, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_pass2_m32<32, true, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<32, 0, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<32, 1, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<32, 2, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_pass2_m32<64, false, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_pass2_m32<64, true, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<64, 0, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<64, 1, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<64, 2, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_pass2_m32<128, false, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_pass2_m32<128, true, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<128, 0, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<128, 1, bf16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<128, 2, bf16_t>(const Args &, hipStream_t);
 template int launch_ring_pass2_m32<16, false, f16_t>(const Args &, hipStream_t);
 template int launch_ring_pass2_m32<16, true, f16_t>(const Args &, hipStream_t);
 template int launch_ring_m32<16, 0, f16_t>(const Args &, hipStream_t);
@@ -2516,11 +2544,11 @@ template int launch_ring_pass2_m32<32, true, f16_t>(const Args &, hipStream_t);
 template int launch_ring_m32<32, 0, f16_t>(const Args &, hipStream_t);
 template int launch_ring_m32<32, 1, f16_t>(const Args &, hipStream_t);
 template int launch_ring_m32<32, 2, f16_t>(const Args &, hipStream_t);
-template int launch_ring_pass2_m32<64, false, f16_t>(const Args &, hipStream_t);
-template int launch_ring_pass2_m32<64, true, f16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<64, 0, f16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<64, 1, f16_t>(const Args &, hipStream_t);
-template int launch_ring_m32<64, 2, f16_t>(const Args &, hipStream_t);
+template int launch_ring_pass2_m32<128, false, bf16_t>(const Args &, hipStream_t);
+template int launch_ring_pass2_m32<128, true, bf16_t>(const Args &, hipStream_t);
+template int launch_ring_m32<128, 0, bf16_t>(const Args &, hipStream_t);
+template int launch_ring_m32<128, 1, bf16_t>(const Args &, hipStream_t);
+template int launch_ring_m32<128, 2, bf16_t>(const Args &, hipStream_t);
 template int launch_ring_pass2_m32<128, false, f16_t>(const Args &, hipStream_t);
 template int launch_ring_pass2_m32<128, true, f16_t>(const Args &, hipStream_t);
 template int launch_ring_m32<128, 0, f16_t>(const Args &, hipStream_t);
@@ -2975,31 +3003,62 @@ int ring_geo(RingGeo &g, const s2attn_ring_up_shape *sh)
                 sh->nlon_out_global / sh->pscale_out, 1, sh->pscale_out};
     return S2ATTN_OK;
 }
+// Is the ring step (MODE as launch_ring_s16) the faster one on split products?  Their workgroup of 64 columns waits at two barriers per
+// band of a run, a wavefront of ring_m32_kernel with its 16 columns at none; `full`: the columns fill four fifths of the tiles.
+// us of forward / pass 1 / pass 2 over all chunks, here against there:
+// bf16 (a staged value is one term: one to three matrix instructions of 16 clocks for eight fp32 ones of 32), heads of 17 to 64: always.
+//   721 x 1440, eight heads of 32, four chunks: 1543 / 1828 / 2992, 2199 / 3361 / 5347; 180 x 360 to 360 x 720, four of 64: 409 / 535 / 845,
+//   625 / 860 / 1656; 181 x 360, four of 32, eight chunks (45 columns): 242 / 272 / 275, 262 / 301 / 316.
+// fp16 (two terms: four or five): 721 x 1440 as above: 1953 / 2584 / 3472, 2209 / 3391 / 5361; 361 x 720 to 181 x 360, four of 64, eight
+//   chunks (23 columns): 1390 / 1834 / 1286, 1763 / 2324 / 2084.  Heads of 17 to 32 need full tiles (181 x 360 to 362 x 720, four of 32, 90
+//   columns: 422 / 538 / 887, 337 / 487 / 927).
+// fp32 (three terms: six, and the splitting): full tiles of one column class, in all passes of 33 to 48 channels (a tile of 48 here, of 64
+//   there; 361 x 720, three heads of 40: 399 / 593 / 637, 455 / 681 / 771, but with two classes of 90 columns 532 / 813 / 1096,
+//   439 / 635 / 1106) and in pass 2 of 17 to 32 (721 x 1440 as above: 4343, 4789; eight chunks, radius 1.5 spacings: 1663, 2153).  Forward
+//   and pass 1, whose sums have to agree in every bit, lose there: 2140 + 2886, 1978 + 3003, and 848 + 1130, 728 + 1028.
+//   64 channels: 752 / 931 / 1875, 671 / 1015 / 1189 (361 x 720, four heads).
+// 16 channels: 361 x 720, four heads, fp16: 789 / 966 / 1549, 617 / 898 / 1068; fp32: 670 / 835 / 1491, 443 / 645 / 775.
+template <int MODE, typename T> bool ring_split(const Args &a)
+{
+    if (a.dk_ <= 16 || a.dk_ > 64) return false;
+    const int cols = MODE < 3 ? (a.r_wo + a.r_qps - 1) / a.r_qps : a.r_nkx / a.kps; // local queries, or keys, of a column class
+    const bool full = 5 * cols >= 4 * ((cols + WQ - 1) / WQ * WQ);
+    if (std::is_same<T, bf16_t>::value) return true;
+    if (std::is_same<T, f16_t>::value) return a.dk_ > 32 || full;
+    return full && a.kps == 1 && a.r_qps == 1 && a.dk_ <= 48 && (a.dk_ > 32 || MODE == 3);
+}
 template <int MODE, typename T> int launch_ring_plan_t(const Args &a, hipStream_t st)
 {
-    if (a.dk_ <= 16) return launch_ring_m32<16, MODE, T>(a, st);
-    if (a.dk_ <= 32) return launch_ring_m32<32, MODE, T>(a, st);
-    if (a.dk_ <= 64) return launch_ring_m32<64, MODE, T>(a, st);
-    return launch_ring_m32<128, MODE, T>(a, st);
+    if (ring_split<MODE, T>(a)) {
+        if constexpr (std::is_same<T, float>::value) {
+            if (a.dk_ > 32) return launch_ring_s16<T, 48, true, MODE>(a, st);
+            if constexpr (MODE == 3) return a.dk_ == 32 ? launch_ring_s16<T, 32, false, MODE>(a, st) : launch_ring_s16<T, 32, true, MODE>(a, st);
+        } else {
+            if (a.dk_ <= 32) return launch_ring_s16<T, 32, true, MODE>(a, st);
+            if (a.dk_ <= 48) return launch_ring_s16<T, 48, true, MODE>(a, st);
+            return launch_ring_s16<T, 64, true, MODE>(a, st);
+        }
+    }
+    auto m32 = [&](auto d) {
+        if constexpr (MODE < 3)
+            return launch_ring_m32<decltype(d)::value, MODE, T>(a, st);
+        else
+            return launch_ring_pass2_m32<decltype(d)::value, MODE == 4, T>(a, st);
+    };
+    if (a.dk_ <= 16) return m32(std::integral_constant<int, 16>());
+    if constexpr (!std::is_same<T, bf16_t>::value) { // (16-bit heads of the widths left out here are all on split products)
+        if (a.dk_ <= 32) return m32(std::integral_constant<int, 32>());
+    }
+    if constexpr (std::is_same<T, float>::value) {
+        if (a.dk_ <= 64) return m32(std::integral_constant<int, 64>());
+    }
+    return m32(std::integral_constant<int, 128>());
 }
 template <int MODE> int launch_ring_plan(const Args &a, int dtype, hipStream_t st)
 {
     if (dtype == S2ATTN_BF16) return launch_ring_plan_t<MODE, bf16_t>(a, st);
     if (dtype == S2ATTN_F16) return launch_ring_plan_t<MODE, f16_t>(a, st);
     return launch_ring_plan_t<MODE, float>(a, st);
-}
-template <bool WRITE, typename T> int launch_ring_pass2_plan_t(const Args &a, hipStream_t st)
-{
-    if (a.dk_ <= 16) return launch_ring_pass2_m32<16, WRITE, T>(a, st);
-    if (a.dk_ <= 32) return launch_ring_pass2_m32<32, WRITE, T>(a, st);
-    if (a.dk_ <= 64) return launch_ring_pass2_m32<64, WRITE, T>(a, st);
-    return launch_ring_pass2_m32<128, WRITE, T>(a, st);
-}
-template <bool WRITE> int launch_ring_pass2_plan(const Args &a, int dtype, hipStream_t st)
-{
-    if (dtype == S2ATTN_BF16) return launch_ring_pass2_plan_t<WRITE, bf16_t>(a, st);
-    if (dtype == S2ATTN_F16) return launch_ring_pass2_plan_t<WRITE, f16_t>(a, st);
-    return launch_ring_pass2_plan_t<WRITE, float>(a, st);
 }
 template <typename SHAPE>
 int ring_forward_plan(const void *k, const void *v, const void *q, float *y_acc, float *alpha_sum, float *qdotk_max, const float *quad_weights,
@@ -3028,7 +3087,7 @@ int ring_pass2_plan(const void *k, const void *v, const void *q, const void *dy,
     if (!aligned(dk, 16) || !aligned(dv, 16)) return s2attn_fail(S2ATTN_E_UNSUPPORTED, "the band-staged ring steps take 16-byte aligned tensors");
     a.r_asum = const_cast<float *>(alpha_sum), a.r_qmax = const_cast<float *>(qdotk_max), a.r_integral = const_cast<float *>(integral_norm);
     a.dk = dk, a.dv = dv;
-    return launch_ring_pass2_plan<WRITE>(a, g.dtype, static_cast<hipStream_t>(stream));
+    return launch_ring_plan<WRITE ? 4 : 3>(a, g.dtype, static_cast<hipStream_t>(stream));
 }
 } // namespace
 

@@ -71,6 +71,7 @@ __device__ inline void s16_split_blocks(uint4 (&o)[3], const f4v (&x)[2])
 template <typename T> struct S16Piece {
     static constexpr int S = std::is_same<T, f16_t>::value ? 2 : 1;
     u4v r;
+    __device__ inline void zero() { r = u4v{0u, 0u, 0u, 0u}; }
     template <bool PAD> __device__ inline void load(const T *p, int first, int n)
     {
         if (!PAD || first + 8 <= n) {
@@ -93,6 +94,7 @@ template <typename T> struct S16Piece {
 template <> struct S16Piece<float> {
     static constexpr int S = 3;
     f4a a, b;
+    __device__ inline void zero() { a = b = f4a{0.f, 0.f, 0.f, 0.f}; }
     template <bool PAD> __device__ inline void load(const float *p, int first, int n)
     {
         a = b = f4a{0.f, 0.f, 0.f, 0.f};
@@ -142,6 +144,26 @@ template <typename T, int D, bool PAD> struct SplitBand {
                 if (W < FRESH) col = min(col, col - (unsigned)W), col = min(col, col - (unsigned)W);
                 ra[it].template load<PAD>(pa + col * lda, ch, na);
                 rb[it].template load<PAD>(pb + col * ldb, ch, nb);
+            }
+        }
+    }
+    // The same for rows lo .. hi of N, zeros elsewhere (a ring step's band is clipped): row lo is column `col` of pa, pb, columns ld elements
+    // apart; wrap > 0: the number of columns the later rows wrap around (at least 32; col + hi - lo < 4 wrap)
+    template <int N> __device__ inline void fetch_rows(const T *pa, const T *pb, int tid, int lo, int hi, unsigned ld, int n, int col = 0, int wrap = 0)
+    {
+        const int r0 = tid / CPR, ch = 8 * (tid % CPR);
+#pragma unroll
+        for (int it = 0; it < (N + RPI - 1) / RPI; it++) {
+            if ((it + 1) * RPI <= N || it * RPI + r0 < N) {
+                const int r = it * RPI + r0;
+                ra[it].zero();
+                rb[it].zero();
+                if (r >= lo && r < hi) {
+                    unsigned x = (unsigned)(col + r - lo);
+                    if (wrap) x = min(x, x - (unsigned)wrap), x = min(x, x - (unsigned)wrap), x = min(x, x - (unsigned)wrap);
+                    ra[it].template load<PAD>(pa + (size_t)x * ld, ch, n);
+                    rb[it].template load<PAD>(pb + (size_t)x * ld, ch, n);
+                }
             }
         }
     }
