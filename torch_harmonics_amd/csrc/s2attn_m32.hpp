@@ -948,7 +948,7 @@ template <int D, bool WRITE, typename T> __global__ __launch_bounds__(64) void r
     const float lw = fast_log2(a.quad_w[hreal + a.r_wlat0]);
 
     Tile qt, gt;
-    float2 st = make_float2(0.f, 0.f);
+    float st_a = 0.f, st_m = 0.f, st_i = 0.f; // alpha_sum, qdotk_max, integral_norm of a staged row, as loaded: first used in commit
     const int r0 = lane / Tile::CPR;
     const unsigned pc = 4u * sizeof(T) * (lane % Tile::CPR);
     const bool piece_ok = 4 * (lane % Tile::CPR) < dr; // this lane's four channels of a staged row exist
@@ -974,14 +974,13 @@ template <int D, bool WRITE, typename T> __global__ __launch_bounds__(64) void r
                 gt.raw[it] = m32_piece<T>(gy + o);
             }
         }
-        if (lane < HK) { // lanes 0..31 fetch the statistics of the staged rows: (log2-sum-exp, integral_norm)
-            st = make_float2(INFINITY, 0.f); // exp2(-inf) = 0
+        if (lane < HK) { // lanes 0..31 fetch the statistics of the staged rows
+            st_a = 0.f;
             if (lane < nrows) {
                 int cr = wk.col + lane;
                 cr -= (cr >= a.Wi) ? a.Wi : 0;
                 const size_t s = sbase + lat + (size_t)cr * a.r_qps;
-                const float as = a.r_asum[s];
-                if (as > 0.f) st = make_float2(fmaf(a.r_qmax[s], LOG2E, fast_log2(as)), a.r_integral[s]); // (a query that saw nothing weighs nothing)
+                st_a = a.r_asum[s], st_m = a.r_qmax[s], st_i = a.r_integral[s];
             }
         }
     };
@@ -989,8 +988,9 @@ template <int D, bool WRITE, typename T> __global__ __launch_bounds__(64) void r
         qt.commit(Qs, lane);
         gt.commit(Gs, lane);
         if (lane < HK) {
-            Ls[lane] = st.x;
-            Is[lane] = st.y;
+            // log2-sum-exp and integral_norm; a query that saw nothing, or a row outside the window, weighs exp2(-inf) = 0
+            Ls[lane] = st_a > 0.f ? fmaf(st_m, LOG2E, fast_log2(st_a)) : INFINITY;
+            Is[lane] = st_a > 0.f ? st_i : 0.f;
         }
     };
     if (any) {
