@@ -436,7 +436,7 @@ template <bool FULL, typename TO> __device__ inline void store_block(TO *dst, co
 // Which operand supplies the rows of the result decides what a lane holds of it: always one index that is contiguous in the
 // destination per lane (32 lanes = 128 bytes of fp32), so stores are coalesced without a detour through LDS.
 template <bool CM, typename TI, typename C, typename TO, int WO, int WN, int NF>
-__global__ __launch_bounds__(64 * WO * WN, 2) void proj_kernel(const ProjArgs a)
+__global__ __launch_bounds__(64 * WO * WN, C::NT == 1 && WO * WN == 8 && NF == 2 ? 4 : 2) void proj_kernel(const ProjArgs a)
 {
     constexpr int NWV = WO * WN, NTILE = 32 * NF * WN, KS = C::KC / 16, NT = C::NT, NBUF = 3;
     constexpr bool DEEP = !CM && NT == 1 && NF == 4;
@@ -887,9 +887,12 @@ template <bool CM, typename TI, typename C, typename TO> int launch_proj(ProjArg
     const int64_t tiles = batch * ((a.points + 127) / 128);
     int wo = a.nblocks >= 3 ? 4 : a.nblocks;
     // 16-bit products: the packed weights come through the vector L1 (64 bytes per clock), which a wavefront's 64 x 64 results use
-    // up; 64 x 128 halve that
+    // up; 64 x 128 halve that.  A channel-major fp32 source of few channels is the exception: its workgroups are over after a few trips to
+    // memory, and two of 64 x 64 per CU overlap theirs (256 channels, 721 x 1440: 1097 -> 1043 .. 1082 us; 192, 181 x 360, batch 2: 106 -> 93;
+    // a point-major 16-bit source of 256: 338 against 290)
+    constexpr bool LATENCY = CM && sizeof(TI) == 4;
     if constexpr (C::NT == 1)
-        if (wo == 4 && tiles / 2 * ((a.nblocks + 3) / 4) >= 512) return launch_tile<CM, TI, C, TO, 4, 2, 4>(a, batch, s);
+        if (wo == 4 && !(LATENCY && a.nchunks <= 4) && tiles / 2 * ((a.nblocks + 3) / 4) >= 512) return launch_tile<CM, TI, C, TO, 4, 2, 4>(a, batch, s);
     while (wo > 1 && tiles * ((a.nblocks + wo - 1) / wo) < 256) wo >>= 1;
     switch (wo) {
     case 4: return launch_tile<CM, TI, C, TO, 4, 2, 2>(a, batch, s);
