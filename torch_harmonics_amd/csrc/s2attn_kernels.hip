@@ -3005,7 +3005,8 @@ int ring_geo(RingGeo &g, const s2attn_ring_up_shape *sh)
 }
 // Is the ring step (MODE as launch_ring_s16) the faster one on split products?  Their workgroup of 64 columns waits at two barriers per
 // band of a run, a wavefront of ring_m32_kernel with its 16 columns at none; `full`: the columns fill four fifths of the tiles.
-// us of forward / pass 1 / pass 2 over all chunks, here against there:
+// us of forward / pass 1 / pass 2 over all chunks, here against there, pass 2 without the early exit of ring_window_seen on either side
+// (it takes a tenth to a quarter off both):
 // bf16 (a staged value is one term: one to three matrix instructions of 16 clocks for eight fp32 ones of 32), heads of 17 to 64: always.
 //   721 x 1440, eight heads of 32, four chunks: 1543 / 1828 / 2992, 2199 / 3361 / 5347; 180 x 360 to 360 x 720, four of 64: 409 / 535 / 845,
 //   625 / 860 / 1656; 181 x 360, four of 32, eight chunks (45 columns): 242 / 272 / 275, 262 / 301 / 316.

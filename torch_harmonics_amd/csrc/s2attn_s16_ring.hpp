@@ -5,8 +5,8 @@
 //
 // What bounds a ring step: on long runs the matrix and vector work of its tile steps, on short ones a run's chain of loads, barrier and
 // one or two steps; the caller's state is read and written once.  All three passes: 721 x 1440, eight heads of 32, four chunks, bf16: 10.9 ms
-// with fp32 matrix instructions on widened values, 6.3 here; 361 x 720, two batches of four heads of 64, radius 0.044, two chunks: 16.9 ms,
-// 6.2 here.  State and gradients are as close to float64 as there or closer (relative 2-norm of y_acc 2.7e-7 for 3.1e-7, dk 2.1e-7 for 2.3e-7).
+// with fp32 matrix instructions on widened values, 5.6 here; 361 x 720, two batches of four heads of 64, radius 0.044, two chunks: 16.9 ms,
+// 6.1 here.  State and gradients are as close to float64 as there or closer (relative 2-norm of y_acc 2.7e-7 for 3.1e-7, dk 2.1e-7 for 2.3e-7).
 //
 // A workgroup of four wavefronts owns 64 consecutive longitudes.  Row x of its band of a run is the grid point "workgroup's first
 // longitude + run start + x"; the chunk (pass 2: the window of local queries) clips ROWS, so of a run's band up to three intervals
@@ -379,7 +379,7 @@ template <typename T, int D, bool PAD, bool WRITE> __global__ __launch_bounds__(
     SplitRingWalk2 wk;
     wk.W = a.Wi, wk.wg0 = wg0, wk.qps = a.r_qps, wk.wo = a.r_wo;
     wk.start(a.sruns, a.soff[hv], a.soff[hv + 1]);
-    const bool any = wk.advance(); // false: none of the queries that see these keys is local
+    const bool any = ring_window_seen(a.sruns, a.soff[hv], a.soff[hv + 1], lane, wg0, WQ, a.Wi, a.r_qps, a.r_wo) && wk.advance(); // false: none of the queries that see these keys is local
     if (!WRITE && !any) return;
 
     const size_t sbase = (size_t)b * (a.Ho / a.r_qps) * a.r_wo; // first local query of the batch entry
