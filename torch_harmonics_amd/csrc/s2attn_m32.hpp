@@ -1,4 +1,5 @@
-// Matrix-core kernels for fp32 storage and head dims 64 / 128: forward, dq and dk/dv with v_mfma_f32_16x16x4_f32.
+// Matrix-core kernels with v_mfma_f32_16x16x4_f32: forward, dq and dk/dv for fp32 heads of up to 16 channels (where s16_faster says so) and of
+// 65 to 512, and the ring steps that ring_split leaves here.
 // Included by s2attn_kernels.hip inside namespace s2 after s2attn_h16.hpp, whose tiling they share: one wavefront owns
 // HQ = 16 consecutive longitudes of one latitude for one (batch, head) and walks every run of that latitude in steps of
 // HK = 32 band positions; lane l = (c = l % 16, qd = l / 16); scores are produced transposed, S^T[position][column].
