@@ -888,6 +888,7 @@ struct RingWalk2 {
 // run.  Band position 0 of run (ws, len) is query column c0, the window holds columns 0 .. nv of the run's class: the band of
 // len + tile - 1 positions meets it iff it starts inside or reaches column 0 again.  Pass 2 over all chunks, us: 721 x 1440, eight heads of 32,
 // four chunks: 4333 -> 3573, bf16 2996 -> 2253; 361 x 720, four heads of 16, three chunks: 768 -> 619, of 64, four chunks: 1113 -> 1016.
+// Up-sampling steps do without: their tiles have zeros to write anyway (180 x 360 to 362 x 720, heads of 32, fp16: 879 with it, 850 without).
 __device__ inline bool ring_window_seen(const Run *runs, int ri, int rend, int lane, int w0, int tile, int W, int qps, int wo)
 {
     for (int i = ri; i < rend; i += 64) {
@@ -935,7 +936,7 @@ template <int D, bool WRITE, typename T> __global__ __launch_bounds__(64) void r
     const bool mine = c < nvalid;
     const size_t pt = ((size_t)b * a.r_nlat + rl) * a.r_nkx + (size_t)((w0 + (mine ? c : 0)) * a.kps + par - a.r_lon_lo); // the key in the chunk
     const int ri = a.soff[hv], rend = a.soff[hv + 1];
-    if (!ring_window_seen(a.sruns, ri, rend, lane, w0, HQ, a.Wi, a.r_qps, a.r_wo)) { // no local query sees these keys
+    if (WRITE ? ri >= rend : !ring_window_seen(a.sruns, ri, rend, lane, w0, HQ, a.Wi, a.r_qps, a.r_wo)) { // no local query sees these keys
         if (WRITE && mine) {
             float *dk = static_cast<float *>(a.dk) + pt * drt + 4 * qd, *dv = static_cast<float *>(a.dv) + pt * drt + 4 * qd;
 #pragma unroll

@@ -379,7 +379,7 @@ template <typename T, int D, bool PAD, bool WRITE> __global__ __launch_bounds__(
     SplitRingWalk2 wk;
     wk.W = a.Wi, wk.wg0 = wg0, wk.qps = a.r_qps, wk.wo = a.r_wo;
     wk.start(a.sruns, a.soff[hv], a.soff[hv + 1]);
-    const bool any = ring_window_seen(a.sruns, a.soff[hv], a.soff[hv + 1], lane, wg0, WQ, a.Wi, a.r_qps, a.r_wo) && wk.advance(); // false: none of the queries that see these keys is local
+    const bool any = (WRITE || ring_window_seen(a.sruns, a.soff[hv], a.soff[hv + 1], lane, wg0, WQ, a.Wi, a.r_qps, a.r_wo)) && wk.advance(); // false: none of the queries that see these keys is local
     if (!WRITE && !any) return;
 
     const size_t sbase = (size_t)b * (a.Ho / a.r_qps) * a.r_wo; // first local query of the batch entry
