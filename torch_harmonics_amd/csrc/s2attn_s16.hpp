@@ -342,7 +342,7 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
     S16Sum acc[NCB]; // Y^T: register v of block cb is channel 16 cb + 4 qd + v of column c
     s16_zero(acc);
     float m = 0.f, Z = 0.f;
-    bool first = true;
+    bool first = true; // this column has seen no neighbor of positive weight
 
     H16Walk wk;
     wk.ri = a.goff[ho];
@@ -386,17 +386,18 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
             float mx = fmaxf(fmaxf(fmaxf(p[0][0], p[0][1]), fmaxf(p[0][2], p[0][3])), fmaxf(fmaxf(p[1][0], p[1][1]), fmaxf(p[1][2], p[1][3])));
             // The running maximum is only the reference point of the exponentials: it moves when a column's maximum has
             // grown by more than RESCALE_THR (probabilities stay below 2^RESCALE_THR), which after a row's first steps is rare.
-            // The first step of a row always sets it (every column has a neighbor in the first step of a run).
-            if (first || __any(mx > RESCALE_THR)) {
+            // A column's first step with a neighbor always sets it.  (Every column has a neighbor in the first step of a run, but on a
+            // latitude of quadrature weight 0 its maximum is -inf, which is no reference point.)
+            if (__any(first || mx > RESCALE_THR)) {
                 const float cm = h16_quarter_max(mx);
-                const float d = first || cm > RESCALE_THR ? cm : 0.f;
+                const float d = (first && cm > -INFINITY) || cm > RESCALE_THR ? cm : 0.f;
                 const float corr = first ? 0.f : fast_exp2(-d);
                 Z *= corr;
 #pragma unroll
                 for (int cb = 0; cb < NCB; cb++) acc[cb].hi *= corr, acc[cb].lo *= corr;
                 p[0] -= d, p[1] -= d;
                 m += d;
-                first = false;
+                first = first && !(cm > -INFINITY);
             }
 #pragma unroll
             for (int kb = 0; kb < 2; kb++) {
