@@ -13,6 +13,7 @@ from typing import Optional, Tuple, Union
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch._C._functorch import maybe_current_level
 
 from ._attention_utils import _check_dtypes_match, _check_extent, _check_ndim
 from ._layout import to_nchw, to_nhwc
@@ -440,9 +441,11 @@ class NeighborhoodAttentionS2(nn.Module):
 
     def _native_dtype(self, query, key, value) -> Optional[torch.dtype]:
         """Element type in which the layer runs as one native operator, None where it is composed of separate operators instead: with a
-        tensor as softmax scale or another attention_handle, for fp64, for tensors that are not plain GPU tensors, and for mixtures
-        of types that torch itself would refuse."""
+        tensor as softmax scale or another attention_handle, for fp64, for tensors that are not plain GPU tensors, inside a functorch
+        transform, and for mixtures of types that torch itself would refuse."""
         if self.attention_handle is not neighborhood_s2_attention or not isinstance(self.scale, (int, float)):
+            return None
+        if not torch.compiler.is_compiling() and maybe_current_level() is not None:  # (wrapped tensors look plain from here)
             return None
         dev, dtype, wdtype = query.device, query.dtype, self.q_weights.dtype
         for t in (query, key, value):

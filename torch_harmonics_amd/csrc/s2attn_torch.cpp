@@ -14,6 +14,8 @@
 // kernels and the autograd rules are registered from Python (torch_harmonics_amd/ops.py), as the reference does.
 
 #include <ATen/ATen.h>
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -622,6 +624,33 @@ void layer_backward(const Tensor &grad, const Tensor *t, const LayerConfig &cfg,
     gr.finish();
 }
 
+#define LAYER_ARGS                                                                                                                                             \
+    const Tensor &query, const c10::optional<Tensor> &key, const c10::optional<Tensor> &value, const Tensor &wq, const Tensor &wk, const Tensor &wv,            \
+        const Tensor &wp, const c10::optional<Tensor> &bq, const c10::optional<Tensor> &bk, const c10::optional<Tensor> &bv, const c10::optional<Tensor> &bp,  \
+        const c10::optional<Tensor> &nq, const c10::optional<Tensor> &nk, double scale, const Tensor &quad_weights, const Tensor &col_idx,                     \
+        const Tensor &row_off, const Tensor &plan, c10::ArrayRef<int64_t> plan_header, int64_t num_heads, int64_t nlat_in, int64_t nlon_in,                    \
+        int64_t nlat_out, int64_t nlon_out, at::ScalarType compute
+#define LAYER_TENSORS                                                                                                                                          \
+    {query, key.value_or(Tensor()), value.value_or(Tensor()), wq, wk, wv, wp, bq.value_or(Tensor()), bk.value_or(Tensor()), bv.value_or(Tensor()),             \
+     bp.value_or(Tensor()), nq.value_or(Tensor()), nk.value_or(Tensor()), quad_weights, col_idx, row_off, plan}
+#define LAYER_CONFIG LayerConfig{num_heads, nlat_in, nlon_in, nlat_out, nlon_out, scale, compute, plan_header.vec()}
+
+// (thirteen tensors and no list: an operator that batching transforms can loop over)
+using Tensors13 = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>;
+std::vector<Tensor> layer_forward_op(LAYER_ARGS);
+Tensors13 layer_backward_op(const Tensor &grad, LAYER_ARGS, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &qraw, const Tensor &kraw,
+                            const Tensor &y, const Tensor &lse, std::array<bool, NGRADS> need);
+Tensors13 as_tuple(const Tensor (&g)[NGRADS])
+{
+    return {g[0], g[1], g[2], g[3], g[4], g[5], g[6], g[7], g[8], g[9], g[10], g[11], g[12]};
+}
+
+// Where a dispatch mode (a tracer, a counter, a policy of what is recomputed) is active or a tensor is a wrapper, the layer's two steps
+// go through the dispatcher, as the operators layer_forward and layer_backward: what the node launches by itself nobody would see.
+bool observed(const Tensor &t) { return c10::impl::dispatch_mode_enabled() || (t.defined() && at::isTensorSubclassLike(t)); }
+
+c10::optional<Tensor> given_or_none(const Tensor &t) { return t.defined() ? c10::optional<Tensor>(t) : c10::nullopt; }
+
 struct LayerFunction : public torch::autograd::Function<LayerFunction> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, at::TensorList given, const c10::intrusive_ptr<LayerState> &state, bool need_backward)
     {
@@ -653,7 +682,21 @@ struct LayerFunction : public torch::autograd::Function<LayerFunction> {
         std::array<bool, NGRADS> need;
         for (int i = 0; i < NGRADS; i++) need[i] = state.slot[i] >= 0 && ctx->needs_input_grad(state.slot[i]);
         const auto t = ctx->get_saved_variables();
-        layer_backward(grads[0], t.data(), state.cfg, need, g);
+        if (observed(grads[0])) {
+            static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("s2attn_kernels::layer_backward", "").typed<decltype(layer_backward_op)>();
+            const LayerConfig &c = state.cfg;
+            const c10::optional<Tensor> none;
+            auto kept = [&](int i) { return t[i].defined() ? t[i] : at::empty({0}, t[S_Q].options()); };
+            const Tensors13 r = op.call(grads[0], t[XQ], given_or_none(t[XK]), given_or_none(t[XV]), t[WQ], t[WK], t[WV], t[WP], none, none, none, none,
+                                   given_or_none(t[NQ]), given_or_none(t[NK]), c.scale, t[QUAD], t[COL], t[ROW], t[PLAN], c.plan_header, c.num_heads, c.nlat_in,
+                                   c.nlon_in, c.nlat_out, c.nlon_out, c.compute, kept(S_Q), kept(S_K), kept(S_V), kept(S_QRAW), kept(S_KRAW), kept(S_Y), kept(S_LSE), need);
+            std::apply([&](const auto &...x) {
+                int i = 0;
+                ((need[i] ? (void)(g[i] = x) : (void)0, i++), ...);
+            }, r);
+        } else {
+            layer_backward(grads[0], t.data(), state.cfg, need, g);
+        }
         for (int i = 0; i < NGRADS; i++)
             if (g[i].defined()) result[state.slot[i]] = g[i];
         return result;
@@ -680,21 +723,15 @@ void check_layer(const Tensor (&t)[NTENSORS], const LayerConfig &cfg)
         TORCH_CHECK(!t[i].defined() || (t[i].numel() == want[i - BQ] && t[i].scalar_type() == t[i <= BP ? i - (BQ - WQ) : (int)NQ].scalar_type()), "bias or norm weight of a wrong length or dtype");
 }
 
-#define LAYER_ARGS                                                                                                                                             \
-    const Tensor &query, const c10::optional<Tensor> &key, const c10::optional<Tensor> &value, const Tensor &wq, const Tensor &wk, const Tensor &wv,            \
-        const Tensor &wp, const c10::optional<Tensor> &bq, const c10::optional<Tensor> &bk, const c10::optional<Tensor> &bv, const c10::optional<Tensor> &bp,  \
-        const c10::optional<Tensor> &nq, const c10::optional<Tensor> &nk, double scale, const Tensor &quad_weights, const Tensor &col_idx,                     \
-        const Tensor &row_off, const Tensor &plan, c10::ArrayRef<int64_t> plan_header, int64_t num_heads, int64_t nlat_in, int64_t nlon_in,                    \
-        int64_t nlat_out, int64_t nlon_out, at::ScalarType compute
-#define LAYER_TENSORS                                                                                                                                          \
-    {query, key.value_or(Tensor()), value.value_or(Tensor()), wq, wk, wv, wp, bq.value_or(Tensor()), bk.value_or(Tensor()), bv.value_or(Tensor()),             \
-     bp.value_or(Tensor()), nq.value_or(Tensor()), nk.value_or(Tensor()), quad_weights, col_idx, row_off, plan}
-#define LAYER_CONFIG LayerConfig{num_heads, nlat_in, nlon_in, nlat_out, nlon_out, scale, compute, plan_header.vec()}
-
 // eager mode: one C++ autograd node
 Tensor module_attention(LAYER_ARGS)
 {
     const Tensor t[NTENSORS] = LAYER_TENSORS;
+    if (at::areAnyTensorSubclassLike(at::ArrayRef<Tensor>(t, NTENSORS))) {
+        static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("s2attn_kernels::layer_forward", "").typed<decltype(layer_forward_op)>();
+        return op.call(query, key, value, wq, wk, wv, wp, bq, bk, bv, bp, nq, nk, scale, quad_weights, col_idx, row_off, plan, plan_header, num_heads, nlat_in,
+                       nlon_in, nlat_out, nlon_out, compute)[0];
+    }
     auto state = c10::make_intrusive<LayerState>();
     state->cfg = LAYER_CONFIG;
     check_layer(t, state->cfg);
@@ -723,22 +760,22 @@ std::vector<Tensor> layer_forward_op(LAYER_ARGS)
     return r;
 }
 
-std::vector<Tensor> layer_backward_op(const Tensor &grad, LAYER_ARGS, at::TensorList kept, std::array<bool, NGRADS> need)
+Tensors13 layer_backward_op(const Tensor &grad, LAYER_ARGS, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &qraw, const Tensor &kraw,
+                            const Tensor &y, const Tensor &lse, std::array<bool, NGRADS> need)
 {
     Tensor given[NTENSORS] = LAYER_TENSORS;
     const LayerConfig cfg = LAYER_CONFIG;
     check_layer(given, cfg);
-    TORCH_CHECK(kept.size() == NKEPT, "layer_backward takes the ", NKEPT, " tensors that layer_forward keeps");
     std::vector<Tensor> t(NSAVED);
     for (int i = 0; i < NTENSORS; i++)
         if (given[i].defined()) t[i] = given[i].contiguous();
-    for (int i = 0; i < NKEPT; i++) t[NTENSORS + i] = kept[i];
+    t[S_Q] = q, t[S_K] = k, t[S_V] = v, t[S_QRAW] = qraw, t[S_KRAW] = kraw, t[S_Y] = y, t[S_LSE] = lse;
     Tensor g[NGRADS];
-    for (int i = 0; i < NGRADS; i++) need[i] = need[i] && given[i].defined();
+    for (int i = 0; i < NGRADS; i++) need[i] = need[i] && (given[i].defined() || (i >= BQ && i <= BP)); // (a bias is not looked at)
     layer_backward(grad, t.data(), cfg, need, g);
-    std::vector<Tensor> r;
-    for (const Tensor &x : g) r.push_back(x.defined() ? x : at::empty({0}, query.options()));
-    return r;
+    for (Tensor &x : g)
+        if (!x.defined()) x = at::empty({0}, query.options());
+    return as_tuple(g);
 }
 
 // ---- layout ---------------------------------------------------------------------------------------------------------------
@@ -811,7 +848,9 @@ TORCH_LIBRARY(s2attn_kernels, m)
         "int[] plan_header, int num_heads, int nlat_in, int nlon_in, int nlat_out, int nlon_out, ScalarType compute";
     m.def(("module_attention(" + layer + ") -> Tensor").c_str(), &module_attention);
     m.def(("layer_forward(" + layer + ") -> Tensor[]").c_str(), {at::Tag::pt2_compliant_tag});
-    m.def(("layer_backward(Tensor grad, " + layer + ", Tensor[] kept, bool[13] need) -> Tensor[]").c_str(), {at::Tag::pt2_compliant_tag});
+    std::string thirteen = "Tensor";
+    for (int i = 1; i < NGRADS; i++) thirteen += ", Tensor";
+    m.def(("layer_backward(Tensor grad, " + layer + ", Tensor q, Tensor k, Tensor v, Tensor q_raw, Tensor k_raw, Tensor y, Tensor lse, bool[13] need) -> (" + thirteen + ")").c_str(), {at::Tag::pt2_compliant_tag});
 }
 
 TORCH_LIBRARY_IMPL(s2attn_kernels, CUDA, m)

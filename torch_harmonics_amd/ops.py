@@ -23,6 +23,7 @@ import ctypes
 from typing import List, Optional, Tuple
 
 import torch
+from torch.utils.flop_counter import register_flop_formula
 
 from . import _lib
 from ._attention_utils import _setup_context_attention_backward
@@ -283,8 +284,10 @@ def _(query, key, value, q_weights, k_weights, v_weights, proj_weights, q_bias, 
 
 @torch.library.register_fake("s2attn_kernels::layer_backward")
 def _(grad, *args):
-    tensors, kept, need = args[:_LAYER_TENSORS], args[-2], args[-1]  # noqa: F841
-    return [t.new_empty(t.shape) if n and t is not None else tensors[0].new_empty((0,)) for t, n in zip(tensors, need)]
+    tensors, need = list(args[:_LAYER_TENSORS]), args[-1]
+    for w in range(3, 7):  # (a bias need not be handed over for its gradient)
+        tensors[w + 4] = tensors[w + 4] if tensors[w + 4] is not None else tensors[w].new_empty(tensors[w].shape[:1])
+    return tuple(t.new_empty(t.shape) if n and t is not None else tensors[0].new_empty((0,)) for t, n in zip(tensors, need))
 
 
 def _layer_setup_context(ctx, inputs, output):
@@ -299,7 +302,7 @@ def _layer_backward_rule(ctx, grads):
     if grads[0] is None:
         return (None,) * (_LAYER_TENSORS + 12)
     need = [t is not None and bool(n) for t, n in zip(tensors, ctx.needs_input_grad)]
-    out = layer_backward(grads[0], *tensors, ctx.scale, *geometry, *ctx.rest, list(kept), need)
+    out = layer_backward(grads[0], *tensors, ctx.scale, *geometry, *ctx.rest, *kept, need)
     return (*[g if n else None for g, n in zip(out, need)], *(None,) * 12)
 
 
@@ -308,6 +311,31 @@ torch.library.register_autograd("s2attn_kernels::layer_forward", _layer_backward
 
 def module_attention_traced(*args):
     return layer_forward(*args)[0]
+
+
+# The layer's matrix products for torch.utils.flop_counter (the attention has no formula, alone or in the layer)
+def _layer_products(query, key, value, q_weights, k_weights, v_weights, proj_weights):
+    """Multiply-adds of the four projections, by the argument (query, key, value) whose points they run over."""
+    points = lambda x: x[0] * x[2] * x[3]  # noqa: E731
+    key = key or query
+    value = value or key
+    n = lambda w: w[0] * w[1]  # noqa: E731
+    return points(query) * n(q_weights), points(key) * n(k_weights), points(value) * n(v_weights), points(query) * n(proj_weights)
+
+
+@register_flop_formula(torch.ops.s2attn_kernels.layer_forward)
+def _(query, key, value, q_weights, k_weights, v_weights, proj_weights, *args, out_shape=None, **kwargs) -> int:
+    return 2 * sum(_layer_products(query, key, value, q_weights, k_weights, v_weights, proj_weights))
+
+
+@register_flop_formula(torch.ops.s2attn_kernels.layer_backward)
+def _(grad, *args, out_shape=None, **kwargs) -> int:
+    q, k, v, p = _layer_products(*args[:7])
+    need = args[-1]
+    has_key, has_value = args[1] is not None, args[2] is not None
+    to_input = (need[0], need[1] if has_key else need[0], need[2] if has_value else need[1] if has_key else need[0])
+    through = any(need[:6]) or any(need[7:10]) or any(need[11:])
+    return 2 * (sum(n for n, wanted in zip((q, k, v), to_input) if wanted) + sum(n for n, wanted in zip((q, k, v, p), need[3:7]) if wanted) + (p if through else 0))
 
 
 # Autocast: k, v, q are brought to the active autocast dtype and the op re-entered with autocast off;
