@@ -15,6 +15,7 @@ OPTIONS = {
     "c24h2_nobias": dict(channels=24, bias=False),
     "bf16": dict(dtype=torch.bfloat16),
     "cross": dict(cross=True),
+    "channels_last": dict(layout=torch.channels_last),
 }
 
 
@@ -23,7 +24,7 @@ def layer(request):
     """(f, leaves, y shape): f(*leaves) is the layer on the inputs and parameters in `leaves`."""
     from torch_harmonics_amd import NeighborhoodAttentionS2
 
-    o = dict(channels=64, dtype=torch.float32, cross=False)
+    o = dict(channels=64, dtype=torch.float32, cross=False, layout=torch.contiguous_format)
     o.update({k: v for k, v in OPTIONS[request.param].items() if k in o})
     torch.manual_seed(5)
     kw = {k: v for k, v in OPTIONS[request.param].items() if k not in o}
@@ -35,7 +36,7 @@ def layer(request):
                 p.uniform_(-0.2, 0.2)
     m = m.to(o["dtype"])
     shapes = [(2, o["channels"], *outs)] + ([(2, o["channels"], *ins)] if o["cross"] else [])
-    return m, [torch.randn(s, device="cuda").to(o["dtype"]) for s in shapes]
+    return m, [torch.randn(s, device="cuda").to(o["dtype"]).contiguous(memory_format=o["layout"]) for s in shapes]
 
 
 def _call(m, xs):
@@ -138,3 +139,34 @@ def test_functorch_transforms_are_refused(layer):
         torch.func.vmap(lambda *t: _call(m, t))(*[torch.stack([x, x]) for x in xs])
     with pytest.raises(RuntimeError, match="functorch"):
         torch.func.grad(lambda *t: _call(m, t).float().sum())(*xs)
+
+
+@pytest.mark.parametrize("traced", [False, True], ids=["node", "operators"])
+def test_gradients_of_the_gradients_are_refused(layer, traced):
+    """create_graph=True is taken, and gives the same gradients; differentiating them is an error, with respect to anything they
+    depend on (a penalty on the layer's gradient must not drop out of a loss)."""
+    from torch_harmonics_amd import ops
+
+    m, xs = layer
+    leaves = [x.requires_grad_() for x in xs]
+    if traced:  # as under torch.compile
+        import torch_harmonics_amd.attention as attention
+
+        mp = pytest.MonkeyPatch()
+        mp.setattr(attention, "module_attention", ops.module_attention_traced)
+    try:
+        y = _call(m, leaves)
+    finally:
+        if traced:
+            mp.undo()
+    wrt = [*leaves, *m.parameters()]
+    dy = torch.randn_like(y).requires_grad_()
+    plain = torch.autograd.grad(y, wrt, dy, retain_graph=True)
+    graph = torch.autograd.grad(y, wrt, dy, create_graph=True)
+    for a, b in zip(graph, plain):
+        assert torch.equal(a, b)
+    assert all(g.requires_grad for g in graph)
+    penalty = sum(g.float().square().sum() for g in graph)
+    for x in (leaves[0], m.q_weights, dy):
+        with pytest.raises(RuntimeError, match="cannot be differentiated"):
+            torch.autograd.grad(penalty, x, retain_graph=True)

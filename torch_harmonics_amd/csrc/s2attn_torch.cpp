@@ -656,7 +656,7 @@ struct LayerFunction : public torch::autograd::Function<LayerFunction> {
     {
         Tensor t[NTENSORS], kept[NKEPT];
         for (int i = 0; i < NTENSORS; i++)
-            if (state->slot[i] >= 0) t[i] = given[state->slot[i]].contiguous();
+            if (state->slot[i] >= 0) t[i] = given[state->slot[i]];
         Tensor out = layer_forward(t, state->cfg, need_backward, kept);
         if (need_backward) {
             torch::autograd::variable_list saved(NSAVED);
@@ -677,12 +677,12 @@ struct LayerFunction : public torch::autograd::Function<LayerFunction> {
         for (int s : state.slot) ngiven += s >= 0;
         torch::autograd::variable_list result(ngiven + 2); // + the two arguments that are no tensors
         if (!grads[0].defined()) return result;
-        if (c10::GradMode::is_enabled()) TORCH_WARN_ONCE("NeighborhoodAttentionS2: the gradients of a backward with create_graph=True are not differentiable themselves");
         Tensor g[NGRADS];
         std::array<bool, NGRADS> need;
         for (int i = 0; i < NGRADS; i++) need[i] = state.slot[i] >= 0 && ctx->needs_input_grad(state.slot[i]);
         const auto t = ctx->get_saved_variables();
-        if (observed(grads[0])) {
+        // (create_graph=True: the operator ties the gradients to what they depend on, and refuses to be differentiated)
+        if (observed(grads[0]) || c10::GradMode::is_enabled()) {
             static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("s2attn_kernels::layer_backward", "").typed<decltype(layer_backward_op)>();
             const LayerConfig &c = state.cfg;
             const c10::optional<Tensor> none;
@@ -742,7 +742,7 @@ Tensor module_attention(LAYER_ARGS)
         state->slot[i] = t[i].defined() ? (int)given.size() : -1;
         if (!t[i].defined()) continue;
         need_backward |= t[i].requires_grad();
-        given.push_back(t[i]);
+        given.push_back(t[i].contiguous()); // (a copy belongs to the graph, so it is made ahead of the node)
     }
     return LayerFunction::apply(at::TensorList(given), state, need_backward && c10::GradMode::is_enabled());
 }

@@ -306,6 +306,11 @@ def _layer_backward_rule(ctx, grads):
     return (*[g if n else None for g, n in zip(out, need)], *(None,) * 12)
 
 
+def _no_second_derivative(ctx, *grads):
+    raise RuntimeError("the gradients of NeighborhoodAttentionS2 cannot be differentiated")
+
+
+torch.library.register_autograd("s2attn_kernels::layer_backward", _no_second_derivative, setup_context=_no_context)
 torch.library.register_autograd("s2attn_kernels::layer_forward", _layer_backward_rule, setup_context=_layer_setup_context)
 
 
