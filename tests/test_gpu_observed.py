@@ -170,3 +170,64 @@ def test_gradients_of_the_gradients_are_refused(layer, traced):
     for x in (leaves[0], m.q_weights, dy):
         with pytest.raises(RuntimeError, match="cannot be differentiated"):
             torch.autograd.grad(penalty, x, retain_graph=True)
+
+
+def _layer_args(m, xs, compute):
+    key = None if len(xs) == 1 else xs[1]
+    return (
+        xs[0], key, None, m.q_weights, m.k_weights, m.v_weights, m.proj_weights, m.q_bias, m.k_bias, m.v_bias, m.proj_bias, m.q_norm_weights, m.k_norm_weights, float(m.scale),
+        m.quad_weights, m.psi_col_idx, m.psi_roff_idx, m.psi_plan, m._psi_plan_header, m.num_heads, m.nlat_in, m.nlon_in, m.nlat_out, m.nlon_out, compute,
+    )  # fmt: skip
+
+
+def test_opcheck_of_the_layer(layer):
+    """Schema, fake kernels and autograd registration of both operators, with and without what the backward needs."""
+    from torch_harmonics_amd import ops
+
+    m, xs = layer
+    args = _layer_args(m, [x.requires_grad_() for x in xs], xs[0].dtype)
+    torch.library.opcheck(ops.layer_forward, (*args, True))
+    plain = tuple(a.detach() if isinstance(a, torch.Tensor) else a for a in args)
+    torch.library.opcheck(ops.layer_forward, (*plain, False))
+    out, *kept = ops.layer_forward(*plain, True)
+    torch.library.opcheck(ops.layer_backward, (torch.randn_like(out), *plain, *kept, [a is not None for a in plain[:13]]))
+
+
+@pytest.mark.parametrize("autocast", [None, torch.bfloat16], ids=["", "autocast"])
+def test_compiled_layer(layer, autocast):
+    m, xs = layer
+    torch._dynamo.reset()
+    compiled = torch.compile(m, backend="aot_eager", fullgraph=True)
+    cast = lambda: torch.autocast("cuda", dtype=autocast or torch.bfloat16, enabled=autocast is not None)  # noqa: E731
+    dy = None
+    results = []
+    for f in (m, compiled):
+        leaves = [x.detach().clone().requires_grad_() for x in xs]
+        with cast():
+            y = _call(f, leaves)
+        dy = torch.randn_like(y) if dy is None else dy
+        results.append((y, *torch.autograd.grad(y, [*leaves, *m.parameters()], dy)))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+    with torch.no_grad(), cast():
+        assert torch.equal(_call(compiled, xs), _call(m, xs))
+
+
+@pytest.mark.parametrize("options", [{}, dict(use_qknorm=True)], ids=["plain", "qknorm"])
+def test_compiled_inference_keeps_nothing_for_a_backward(options):
+    from torch_harmonics_amd import NeighborhoodAttentionS2
+
+    torch._dynamo.reset()
+    m = NeighborhoodAttentionS2(64, (32, 64), (32, 64), num_heads=16, theta_cutoff=0.3, **options).cuda().eval()
+    compiled = torch.compile(m, backend="aot_eager", fullgraph=True)
+    x = torch.randn(8, 64, 32, 64, device="cuda")
+    peak = []
+    with torch.no_grad():
+        for f in (m, compiled):
+            f(x)
+            torch.cuda.synchronize()
+            base = torch.cuda.memory_allocated()
+            torch.cuda.reset_peak_memory_stats()
+            f(x)
+            peak.append(torch.cuda.max_memory_allocated() - base)
+    assert peak[1] <= peak[0] + 65536, peak  # (the normaliser alone is 1 MB)

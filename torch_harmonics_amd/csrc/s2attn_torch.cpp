@@ -637,7 +637,7 @@ void layer_backward(const Tensor &grad, const Tensor *t, const LayerConfig &cfg,
 
 // (thirteen tensors and no list: an operator that batching transforms can loop over)
 using Tensors13 = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>;
-std::vector<Tensor> layer_forward_op(LAYER_ARGS);
+std::vector<Tensor> layer_forward_op(LAYER_ARGS, bool keep);
 Tensors13 layer_backward_op(const Tensor &grad, LAYER_ARGS, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &qraw, const Tensor &kraw,
                             const Tensor &y, const Tensor &lse, std::array<bool, NGRADS> need);
 Tensors13 as_tuple(const Tensor (&g)[NGRADS])
@@ -723,6 +723,13 @@ void check_layer(const Tensor (&t)[NTENSORS], const LayerConfig &cfg)
         TORCH_CHECK(!t[i].defined() || (t[i].numel() == want[i - BQ] && t[i].scalar_type() == t[i <= BP ? i - (BQ - WQ) : (int)NQ].scalar_type()), "bias or norm weight of a wrong length or dtype");
 }
 
+bool wants_gradient(const Tensor (&t)[NTENSORS])
+{
+    bool any = false;
+    for (const Tensor &x : t) any |= x.defined() && x.requires_grad();
+    return any && c10::GradMode::is_enabled();
+}
+
 // eager mode: one C++ autograd node
 Tensor module_attention(LAYER_ARGS)
 {
@@ -730,32 +737,30 @@ Tensor module_attention(LAYER_ARGS)
     if (at::areAnyTensorSubclassLike(at::ArrayRef<Tensor>(t, NTENSORS))) {
         static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("s2attn_kernels::layer_forward", "").typed<decltype(layer_forward_op)>();
         return op.call(query, key, value, wq, wk, wv, wp, bq, bk, bv, bp, nq, nk, scale, quad_weights, col_idx, row_off, plan, plan_header, num_heads, nlat_in,
-                       nlon_in, nlat_out, nlon_out, compute)[0];
+                       nlon_in, nlat_out, nlon_out, compute, wants_gradient(t))[0];
     }
     auto state = c10::make_intrusive<LayerState>();
     state->cfg = LAYER_CONFIG;
     check_layer(t, state->cfg);
     std::vector<Tensor> given;
     given.reserve(NTENSORS);
-    bool need_backward = false;
     for (int i = 0; i < NTENSORS; i++) {
         state->slot[i] = t[i].defined() ? (int)given.size() : -1;
         if (!t[i].defined()) continue;
-        need_backward |= t[i].requires_grad();
         given.push_back(t[i].contiguous()); // (a copy belongs to the graph, so it is made ahead of the node)
     }
-    return LayerFunction::apply(at::TensorList(given), state, need_backward && c10::GradMode::is_enabled());
+    return LayerFunction::apply(at::TensorList(given), state, wants_gradient(t));
 }
 
 // the same two steps as operators without an autograd node of their own: what a compiled graph records (fake kernels and the autograd
-// rule in ops.py).  An absent tensor is returned as an empty one.
-std::vector<Tensor> layer_forward_op(LAYER_ARGS)
+// rule in ops.py).  keep: also return what the backward needs.  An absent tensor is returned as an empty one.
+std::vector<Tensor> layer_forward_op(LAYER_ARGS, bool keep)
 {
     const Tensor t[NTENSORS] = LAYER_TENSORS;
     const LayerConfig cfg = LAYER_CONFIG;
     check_layer(t, cfg);
     Tensor kept[NKEPT];
-    std::vector<Tensor> r{layer_forward(t, cfg, true, kept)};
+    std::vector<Tensor> r{layer_forward(t, cfg, keep, kept)};
     for (const Tensor &x : kept) r.push_back(x.defined() ? x : at::empty({0}, query.options().dtype(compute)));
     return r;
 }
@@ -847,7 +852,7 @@ TORCH_LIBRARY(s2attn_kernels, m)
         "Tensor? v_bias, Tensor? proj_bias, Tensor? q_norm, Tensor? k_norm, float scale, Tensor quad_weights, Tensor col_idx, Tensor row_off, Tensor plan, "
         "int[] plan_header, int num_heads, int nlat_in, int nlon_in, int nlat_out, int nlon_out, ScalarType compute";
     m.def(("module_attention(" + layer + ") -> Tensor").c_str(), &module_attention);
-    m.def(("layer_forward(" + layer + ") -> Tensor[]").c_str(), {at::Tag::pt2_compliant_tag});
+    m.def(("layer_forward(" + layer + ", bool keep) -> Tensor[]").c_str(), {at::Tag::pt2_compliant_tag});
     std::string thirteen = "Tensor";
     for (int i = 1; i < NGRADS; i++) thirteen += ", Tensor";
     m.def(("layer_backward(Tensor grad, " + layer + ", Tensor q, Tensor k, Tensor v, Tensor q_raw, Tensor k_raw, Tensor y, Tensor lse, bool[13] need) -> (" + thirteen + ")").c_str(), {at::Tag::pt2_compliant_tag});

@@ -268,14 +268,17 @@ def neighborhood_s2_attention(kw, vw, qw, quad_weights, col_idx, row_off, nh, nl
 
 
 # The layer under torch.compile: the same kernels as module_attention, with fake kernels and an autograd rule the tracer can record.
+_LAYER_KEPT = 7  # what layer_forward returns besides the result: q, k, v, q and k before their norm, y, the softmax normaliser
 _LAYER_TENSORS = 13  # query, key, value, four weights, four biases, two norm gains: the arguments that may need a gradient
 
 
 @torch.library.register_fake("s2attn_kernels::layer_forward")
 def _(query, key, value, q_weights, k_weights, v_weights, proj_weights, q_bias, k_bias, v_bias, proj_bias, q_norm, k_norm, scale, quad_weights, col_idx,
-      row_off, plan, plan_header, num_heads, nlat_in, nlon_in, nlat_out, nlon_out, compute):  # fmt: skip
+      row_off, plan, plan_header, num_heads, nlat_in, nlon_in, nlat_out, nlon_out, compute, keep):  # fmt: skip
     B, ck, cv = query.shape[0], q_weights.shape[0], v_weights.shape[0]
     new = lambda *s: query.new_empty(s, dtype=compute)  # noqa: E731
+    if not keep:
+        return [new(B, cv, nlat_out, nlon_out)] + [new(0) for _ in range(_LAYER_KEPT)]
     q, k = new(B, nlat_out, nlon_out, ck), new(B, nlat_in, nlon_in, ck)
     raw = (new(0), new(0)) if q_norm is None else (torch.empty_like(q), torch.empty_like(k))
     lse = query.new_empty((B, num_heads, nlat_out, nlon_out), dtype=torch.float32)
@@ -292,7 +295,7 @@ def _(grad, *args):
 
 def _layer_setup_context(ctx, inputs, output):
     ctx.save_for_backward(*inputs[:_LAYER_TENSORS], *inputs[14:18], *output[1:])
-    ctx.scale, ctx.rest = inputs[13], inputs[18:]
+    ctx.scale, ctx.rest, ctx.kept = inputs[13], inputs[18:-1], inputs[-1]
     ctx.set_materialize_grads(False)
 
 
@@ -300,10 +303,12 @@ def _layer_backward_rule(ctx, grads):
     saved = ctx.saved_tensors
     tensors, geometry, kept = saved[:_LAYER_TENSORS], saved[_LAYER_TENSORS : _LAYER_TENSORS + 4], saved[_LAYER_TENSORS + 4 :]
     if grads[0] is None:
-        return (None,) * (_LAYER_TENSORS + 12)
+        return (None,) * (_LAYER_TENSORS + 13)
+    if not ctx.kept:
+        raise RuntimeError("layer_forward ran with keep=False: nothing of it is left for a backward")
     need = [t is not None and bool(n) for t, n in zip(tensors, ctx.needs_input_grad)]
     out = layer_backward(grads[0], *tensors, ctx.scale, *geometry, *ctx.rest, *kept, need)
-    return (*[g if n else None for g, n in zip(out, need)], *(None,) * 12)
+    return (*[g if n else None for g, n in zip(out, need)], *(None,) * 13)
 
 
 def _no_second_derivative(ctx, *grads):
@@ -315,7 +320,8 @@ torch.library.register_autograd("s2attn_kernels::layer_forward", _layer_backward
 
 
 def module_attention_traced(*args):
-    return layer_forward(*args)[0]
+    keep = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in args[:_LAYER_TENSORS])
+    return layer_forward(*args, keep)[0]
 
 
 # The layer's matrix products for torch.utils.flop_counter (the attention has no formula, alone or in the layer)
