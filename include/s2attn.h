@@ -29,6 +29,13 @@
  * dq up to 5e-6 beyond 1e-5 on values of magnitude 30-70, as far as a plain fp32 CPU evaluation is off there.  16-bit storage (arithmetic in fp32, P and dS enter the
  * matrix instructions in the storage type): fp16 within 2e-2 |x| + 2e-2 RMS per element; bf16 the same on typical problems, single
  * elements of dq (wide heads) and dk (sums over many queries of both signs) up to 0.2 RMS off in a sweep of random problems.
+ *
+ * Values that are not finite: a NaN or an infinity reaches the points that see it, as arithmetic on each point's neighbors has it, and
+ * no other.  Two kernel families give less: fp32 heads of 32 channels on large grids with mostly short runs, and 16-bit heads of equal
+ * width (a multiple of 8, 16 to 256); there it may also reach points of the same batch entry and head whose neighborhoods share a tile
+ * with the point: at most a tile (32 or 16 longitudes) and a run away in longitude, on the latitudes that see the point's latitude.  A
+ * ring step may pass it to the 16 longitudes of a tile in the same way, and where its fp32 or fp16 operands are split an infinity counts as
+ * NaN.  A quadrature weight of zero takes its latitude out of the softmax; y is NaN where nothing is left.
  */
 #ifndef S2ATTN_H
 #define S2ATTN_H

@@ -1,7 +1,8 @@
 """
-Operands at the edge of their range - quadrature weights of zero - on every kernel family of the attention, against float64.
+Operands at the edge of their range - quadrature weights of zero and below, NaN, infinities, the largest magnitudes - on every
+kernel family of the attention, against float64.
 
-Bounds: fp32 rtol = atol = 1e-5, the suite's bound for fp32; 16-bit storage as in test_gpu_widths._bounds.
+Bounds: fp32 rtol = atol = 1e-5, the suite's bound for fp32; 16-bit storage as in test_gpu_widths._bounds, or 2e-2 of the tensor's scale.
 """
 
 import pytest
@@ -14,8 +15,8 @@ from tests.util import assert_close, randn_inputs
 
 pytestmark = pytest.mark.gpu
 
-# storage, ck, cv, grid (input and output), batch copies, heads.  Copies of one batch entry: the fp32 dispatch goes by the number of
-# workgroups (heads of up to 16 channels: 1024, heads of 32: 4096), the oracle by one entry.
+# storage, ck, cv, grid (one, or input and output grid), batch copies, heads.  Copies of one batch entry: the fp32 dispatch goes by the
+# number of workgroups (heads of up to 16 channels: 1024, heads of 32: 4096), the oracle by one entry.
 SHAPES = {
     "f32_c3c5": (F32, 3, 5, (9, 48), 1, 2),  # vector kernels
     "f32_c8": (F32, 8, 8, (9, 48), 1, 2),  # 16-longitude fp32 tiles, few workgroups
@@ -23,32 +24,43 @@ SHAPES = {
     "f32_c4c12_many": (F32, 4, 12, (9, 48), 60, 2),
     "f32_c16_many": (F32, 16, 16, (9, 48), 60, 2),
     "f32_c20c12": (F32, 20, 12, (9, 48), 1, 2),
+    "f32_c20c12_down": (F32, 20, 12, ((9, 96), (5, 48)), 1, 2),
+    "f32_c20c12_up": (F32, 20, 12, ((5, 34), (9, 102)), 1, 2),
     "f32_c32": (F32, 32, 32, (9, 64), 1, 2),
     "f32_c32_many": (F32, 32, 32, (16, 64), 128, 2),  # hybrid kernels over short runs
     "f32_c40": (F32, 40, 40, (9, 48), 1, 2),
     "f32_c64": (F32, 64, 64, (9, 48), 1, 2),
     "f32_c68c20": (F32, 68, 20, (9, 48), 1, 2),  # fp32 tiles of 128 channels
+    "f32_c68c20_down": (F32, 68, 20, ((9, 96), (5, 48)), 1, 2),
+    "f32_c68c20_up": (F32, 68, 20, ((5, 34), (9, 102)), 1, 2),
     "f32_c160": (F32, 160, 160, (9, 48), 1, 1),  # two channel groups
+    "f32_c20c132": (F32, 20, 132, (9, 48), 1, 1),
     "bf16_c32": (BF16, 32, 32, (9, 48), 1, 2),  # 16-bit tiles
     "bf16_c20c12": (BF16, 20, 12, (9, 48), 1, 2),  # split products
     "bf16_c12": (BF16, 12, 12, (9, 48), 1, 2),
     "f16_c64": (F16, 64, 64, (9, 48), 1, 2),
     "f16_c36c44": (F16, 36, 44, (9, 48), 1, 2),
+    "f16_c36c44_up": (F16, 36, 44, ((5, 34), (9, 102)), 1, 2),
 }
+TILES = {"f32_c32_many", "bf16_c32", "f16_c64"}  # what is not finite may reach the columns of a whole tile
 
 
 def _problem(shape, theta):
-    dtype, ck, cv, (H, W), copies, nh = SHAPES[shape]
-    col, roff = ogeo.neighborhood_csr((H, W), (H, W), "equiangular", "equiangular", theta)
-    quad = ogeo.attention_quad_weights(H, W, "equiangular")
-    k, v, q, dy = [t.to(dtype) for t in randn_inputs(1, H, W, H, W, nh, ck, cv, scale=1.0 if dtype == F32 else 0.5)]
-    return dtype, (k, v, q, dy), quad, col, roff, nh, copies
+    dtype, ck, cv, grid, copies, nh = SHAPES[shape]
+    ins, outs = grid if isinstance(grid[0], tuple) else (grid, grid)
+    up = oracle.is_upsample(ins[1], outs[1])
+    col, roff = ogeo.neighborhood_csr(*((outs, ins) if up else (ins, outs)), "equiangular", "equiangular", theta)
+    quad = ogeo.attention_quad_weights(*ins, "equiangular")
+    mask = (oracle.dense_mask_upsample if up else oracle.dense_mask)(col, roff, *ins, *outs)
+    tensors = [t.to(dtype) for t in randn_inputs(1, *ins, *outs, nh, ck, cv, scale=1.0 if dtype == F32 else 0.5)]
+    return dtype, tensors, quad, (col, roff, nh, copies), mask
 
 
-def _run(tensors, quad, col, roff, nh, copies):
+def _run(tensors, quad, geometry):
     """(y, dk, dv, dq) of the first batch entry; the others are the same entry and have to give the same bits."""
     from torch_harmonics_amd import ops
 
+    col, roff, nh, copies = geometry
     k, v, q, dy = [t.cuda().repeat(copies, 1, 1, 1) for t in tensors]
     geo = (quad.cuda(), col.cuda(), roff.cuda(), nh, k.shape[2], q.shape[1], q.shape[2])
     y, lse = ops.forward_lse(k, v, q, *geo)
@@ -59,13 +71,32 @@ def _run(tensors, quad, col, roff, nh, copies):
     return [t[:1].cpu() for t in out]
 
 
+def _true_neighbors(tensors, quad, mask, nh):
+    """(y, dk, dv, dq) in float64 from each query's true neighbors and nothing else (attention_torch.py:97-125), differentiated by torch."""
+    idx = torch.zeros(mask.shape[0], int(mask.sum(1).max()), dtype=torch.int64)
+    there = torch.zeros(idx.shape, dtype=torch.bool)
+    for i, row in enumerate(mask):
+        n = row.nonzero().flatten()
+        idx[i], idx[i, : len(n)], there[i, : len(n)] = n[0], n, True  # (padded with a true neighbor, which then counts once)
+    k, v, q, dy = tensors
+    leaves = [t.double().requires_grad_(True) for t in (k, v, q)]
+    K, V, Q = [t.reshape(-1, nh, t.shape[3] // nh) for t in leaves]
+    w = quad.double().repeat_interleave(k.shape[2])[idx]
+    s = (Q[:, None] * K[idx]).sum(-1)
+    s = torch.where(there[..., None], s, -torch.inf)
+    p = torch.where(there[..., None], torch.exp(s - torch.nan_to_num(s.detach(), nan=-torch.inf, posinf=torch.inf).amax(1, keepdim=True)) * w[..., None], 0.0)
+    y = sum(torch.where(there[:, i, None, None], p[:, i, :, None] * V[idx[:, i]], 0.0) for i in range(idx.shape[1])) / p.sum(1)[..., None]
+    y = y.reshape(1, q.shape[1], q.shape[2], -1)
+    y.backward(dy.double())
+    return [y.detach()] + [t.grad for t in leaves]
+
+
 @pytest.mark.parametrize("zero", ["first", "middle", "first_two", "all_but_one"])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_quadrature_weight_zero(shape, zero):
     """A latitude of quadrature weight zero takes no part in the softmax, wherever it stands in a query's neighborhood (the reference
     multiplies by the weight, attention_torch.py:97-125).  all_but_one: with a disk that holds the whole sphere."""
-    theta = 4.0 if zero == "all_but_one" else 0.9
-    dtype, tensors, quad, col, roff, nh, copies = _problem(shape, theta)
+    dtype, tensors, quad, geometry, mask = _problem(shape, 4.0 if zero == "all_but_one" else 0.9 if SHAPES[shape][3][0] in (9, 16) or isinstance(SHAPES[shape][3][0], tuple) and SHAPES[shape][3][0][0] == 9 else 1.7)
     H = quad.numel()
     quad = quad.clone()
     quad[{"first": slice(0, 1), "middle": slice(H // 2, H // 2 + 1), "first_two": slice(0, 2), "all_but_one": slice(0, H - 2)}[zero]] = 0.0
@@ -73,16 +104,57 @@ def test_quadrature_weight_zero(shape, zero):
         quad[H - 1] = 0.0
     k, v, q, dy = tensors
     kr, vr, qr = [t.double().requires_grad_(True) for t in (k, v, q)]
-    y64 = oracle.dense_attention_f64(kr, vr, qr, quad, col, roff, nh)
+    y64 = oracle.dense_attention_f64(kr, vr, qr, quad, *geometry[:3])
     assert torch.isfinite(y64).all(), "every query is left a neighbor"
     y64.backward(dy.double())
     want = [y64.detach(), kr.grad, vr.grad, qr.grad]
-    got = _run(tensors, quad, col, roff, nh, copies)
+    got = _run(tensors, quad, geometry)
     if dtype == F32:
         for name, a, b in zip(("y", "dk", "dv", "dq"), got, want):
             assert_close(name, a, b, rtol=1e-5, atol=1e-5)
         return
-    mask = oracle.dense_mask(col, roff, H, k.shape[2], H, k.shape[2])
-    for name, a, b, bound in zip(("y", "dk", "dv", "dq"), got, want, _bounds(k, v, q, dy, quad, mask, nh, 2.0**-8 if dtype == BF16 else 2.0**-11)):
+    for name, a, b, bound in zip(("y", "dk", "dv", "dq"), got, want, _bounds(k, v, q, dy, quad, mask, geometry[2], 2.0**-8 if dtype == BF16 else 2.0**-11)):
         worst = ((a.double() - b).abs() - bound).max().item()
         assert torch.isfinite(a).all() and worst <= 0, f"{name}: {worst:.3e} beyond the bound"
+
+
+NAN, INF = float("nan"), float("inf")
+POISON = {"k_nan": (0, NAN), "v_nan": (1, NAN), "q_nan": (2, NAN), "dy_nan": (3, NAN), "k_minus_inf": (0, -INF), "v_inf": (1, INF), "dy_inf": (3, -INF), "v_huge": (1, 3.4e38)}
+
+
+@pytest.mark.parametrize("poison", [*POISON, "weight_below_zero"])
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s not in TILES])
+def test_what_is_not_finite_reaches_true_neighbors_only(shape, poison):
+    """One channel of one point is NaN, infinite or of a magnitude that only fp32 holds: what sees the point gets what float64
+    arithmetic on its neighbors gives, and everything else the result it has without it."""
+    dtype, tensors, quad, geometry, mask = _problem(shape, 0.6 if SHAPES[shape][3][0] in (9, 16) or isinstance(SHAPES[shape][3][0], tuple) and SHAPES[shape][3][0][0] == 9 else 0.9)
+    if poison == "weight_below_zero":
+        quad = quad.clone()
+        quad[quad.numel() // 2] *= -0.01  # (the sums must not cancel)
+    else:
+        which, value = POISON[poison]
+        if dtype != F32 and poison == "v_huge":
+            pytest.skip("fp32's range")
+        t = tensors[which]
+        t[0, t.shape[1] // 2, t.shape[2] // 3, 1] = value
+    got, want = _run(tensors, quad, geometry), _true_neighbors(tensors, quad, mask, geometry[2])
+    clean = (poison == "weight_below_zero") or None
+    for name, a, b in zip(("y", "dk", "dv", "dq"), got, want):
+        if poison == "v_huge" and name != "y":  # (<dy, v> leaves fp32's range)
+            continue
+        a = a.double()
+        finite = torch.isfinite(b)
+        assert bool(finite.all()) if clean else True
+        assert torch.equal(torch.isfinite(a), finite), f"{name}: {int((torch.isfinite(a) != finite).sum())} of {finite.numel()} values are finite on one side only"
+        if name == "y":
+            special = lambda x: torch.nan_to_num(x, nan=7.0, posinf=8.0, neginf=9.0)  # noqa: E731
+            assert torch.equal(special(a)[~finite], special(b)[~finite])
+        if name == "y" and poison == "v_huge":
+            big = b.abs() > 1e30
+            assert_close(name, a[big] / 1e38, b[big] / 1e38, rtol=1e-5, atol=0)
+            finite &= ~big
+        x, y = a[finite], b[finite]
+        if dtype == F32:
+            assert_close(name, x, y, rtol=1e-5, atol=1e-5)
+        else:
+            assert_close(name, x, y, rtol=2e-2, atol=2e-2 * y.square().mean().sqrt().item())

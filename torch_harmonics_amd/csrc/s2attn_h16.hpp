@@ -236,8 +236,9 @@ __device__ inline void xcd_split(int id, int BH, int per_bh, int &bh, int &rest)
     }
 }
 
-#define S2_H16_IDS(W_TILED, NROWS)                                            \
-    const int tid = threadIdx.x;                                              \
+#define S2_H16_IDS(W_TILED, NROWS) S2_H16_IDS_OF(threadIdx.x, W_TILED, NROWS)
+#define S2_H16_IDS_OF(TID, W_TILED, NROWS)                                    \
+    const int tid = TID;                                                      \
     const int lane = tid & 63, wave = tid >> 6;                               \
     const int c = lane & 15, qd = lane >> 4;                                  \
     const int BH = a.B * a.nh;                                                \

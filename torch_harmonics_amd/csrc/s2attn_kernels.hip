@@ -289,6 +289,8 @@ template <int P> __device__ inline float dot_row(const float (&a)[P], const floa
 
 struct PRun;
 
+enum Which { FWD, DQ, DKDV }; // the three passes
+
 struct Args {
     const void *k, *v, *q, *dy;
     void *y, *dk, *dv, *dq;
@@ -2277,6 +2279,7 @@ template <typename T> __global__ __launch_bounds__(64) void dkdv_mfma_kernel(con
 }
 
 #include "s2attn_h16.hpp"
+#include "s2attn_points.hpp"
 #include "s2attn_m32.hpp"
 #include "s2attn_s16.hpp"
 #include "s2attn_s16_ring.hpp"
@@ -2311,8 +2314,6 @@ template <typename E> __global__ __launch_bounds__(256) void transpose_kernel(co
 // shape the dispatch below names) in their own compilation of this file
 // ---------------------------------------------------------------------------------
 namespace s2 {
-
-enum Which { FWD, DQ, DKDV };
 
 template <typename T, int D, bool PAD> int launch_h16(Which which, const Args &a0, hipStream_t stream);
 template <int D, int NS> int launch_m32(Which which, const Args &a0, hipStream_t stream);

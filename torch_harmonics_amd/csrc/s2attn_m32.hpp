@@ -20,8 +20,9 @@
 // tiles, operands and output channels); the partial scores of the groups are added through LDS once per step, after which
 // both wavefronts hold the same probabilities.  One wavefront cannot hold a 256-channel step in registers.
 
-#define S2_M32_IDS(W_TILED, NROWS)                                            \
-    const int lane = NS > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;     \
+#define S2_M32_IDS(W_TILED, NROWS) S2_M32_IDS_OF(NS > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x, W_TILED, NROWS)
+#define S2_M32_IDS_OF(LANE, W_TILED, NROWS)                                   \
+    const int lane = LANE;                                                    \
     const int wv = NS > 1 ? (int)(threadIdx.x >> 6) : 0;                      \
     const int c = lane & 15, qd = lane >> 4;                                  \
     const int BH = a.B * a.nh;                                                \
@@ -175,6 +176,21 @@ template <typename T> __device__ inline u4v m32_piece(const char *p)
     return u4v{__float_as_uint(x.x), __float_as_uint(x.y), __float_as_uint(x.z), __float_as_uint(x.w)};
 }
 
+// The columns `redo` of a wavefront whose sums are not finite: its own channel group of them (see s2attn_points.hpp)
+template <int D, int NS, Which PASS> __device__ inline void m32_points(unsigned redo)
+{
+    const Args a = point_args();
+    S2_M32_IDS_OF(point_lane(), PASS == DKDV ? a.Wi : a.Wo, PASS == DKDV ? a.Hi : a.Ho)
+    (void)c, (void)qd, (void)nvalid, (void)ldbk_, (void)ldbv_;
+    const int row = (PASS == DKDV ? a.sorder : a.gorder)[a.row_first + rowsel];
+    for (; redo; redo &= redo - 1) {
+        const int col = w0 + __builtin_ctz(redo);
+        if (PASS == FWD) point_forward<float, D / 16>(a, b, h, bh, row, col, cbase, nv, wv == 0, lane);
+        if (PASS == DQ) point_dq<float, D / 16>(a, b, h, bh, row, col, cbase, nk, false, lane);
+        if (PASS == DKDV) point_dkdv<float, D / 16>(a, b, h, bh, row, col, cbase, nk, nv, lane);
+    }
+}
+
 // ---- forward ---------------------------------------------------------------------------------------------------
 template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kernel(const Args a)
 {
@@ -292,7 +308,11 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kern
     }
 
     S = h16_quarter_sum(S);
-    if (mine) {
+    float check = S;
+#pragma unroll
+    for (int cb = 0; cb < NCB; cb++) check += point_sum(acc[cb]);
+    const unsigned redo = point_columns(mine && not_finite(check));
+    if (mine && !(redo >> c & 1)) {
         if (a.lse && qd == 0 && wv == 0) a.lse[((size_t)bh * a.Ho + ho) * a.Wo + w0 + c] = m + fast_log2(S);
         const float inv = 1.0f / S;
         char *y = static_cast<char *>(a.y) + pt * ldbv_ + (size_t)h * (a.dv_ * 4) + cbase * 4 + 16 * qd;
@@ -301,6 +321,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kern
             if (16 * cb + 4 * qd < nv)
                 *reinterpret_cast<float4 *>(y + 64 * cb) = make_float4(acc[cb][0] * inv, acc[cb][1] * inv, acc[cb][2] * inv, acc[cb][3] * inv);
     }
+    if (redo) m32_points<D, NS, FWD>(redo);
 }
 
 // ---- backward, dq pass (needs the forward's y and lse) -------------------------------------------------------------
@@ -426,13 +447,18 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dq_m32_kerne
 
     // (stored after the walk: a global store ahead of the loop would turn the loop's scalar loads of runs and weights,
     // which the compiler only uses while nothing in the kernel can have written memory, into vector loads with waits)
+    float check = 0.f;
+#pragma unroll
+    for (int cb = 0; cb < NCB; cb++) check += point_sum(acc[cb]);
+    const unsigned redo = point_columns(mine && not_finite(check));
     if (mine && qd == 0 && wv == 0) a.stats[sidx] = make_float2(lse, I);
-    if (mine) {
+    if (mine && !(redo >> c & 1)) {
         char *dq = static_cast<char *>(a.dq) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4 + 16 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++)
             if (16 * cb + 4 * qd < nk) *reinterpret_cast<float4 *>(dq + 64 * cb) = make_float4(acc[cb][0], acc[cb][1], acc[cb][2], acc[cb][3]);
     }
+    if (redo) m32_points<D, NS, DQ>(redo);
 }
 
 // ---- backward, dk/dv pass: transposed gather ---------------------------------------------------------------------
@@ -550,7 +576,11 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dkdv_m32_ker
         run = nrun;
     }
 
-    if (mine) {
+    float check = 0.f;
+#pragma unroll
+    for (int cb = 0; cb < NCB; cb++) check += point_sum(dkt[cb] + dvt[cb]);
+    const unsigned redo = point_columns(mine && not_finite(check));
+    if (mine && !(redo >> c & 1)) {
         char *dk = static_cast<char *>(a.dk) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4 + 16 * qd;
         char *dv = static_cast<char *>(a.dv) + pt * ldbv_ + (size_t)h * (a.dv_ * 4) + cbase * 4 + 16 * qd;
 #pragma unroll
@@ -559,6 +589,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dkdv_m32_ker
             if (16 * cb + 4 * qd < nv) *reinterpret_cast<float4 *>(dv + 64 * cb) = make_float4(dvt[cb][0], dvt[cb][1], dvt[cb][2], dvt[cb][3]);
         }
     }
+    if (redo) m32_points<D, NS, DKDV>(redo);
 }
 
 // ---- forward, one ring step --------------------------------------------------------------------------------------

@@ -320,6 +320,21 @@ template <typename T, int D> constexpr int s16_lds_bytes(bool stats) { return 2 
 // block of the ring `n` blocks after block `first` (both below 5)
 __device__ inline int s16_block(int first, int n) { return first + n >= FRESH / 16 ? first + n - FRESH / 16 : first + n; }
 
+// The columns `redo` of a wavefront whose sums are not finite (see s2attn_points.hpp)
+template <typename T, int N, Which PASS> __device__ inline void s16_points(unsigned redo, int wv)
+{
+    const Args a = point_args();
+    S2_H16_IDS_OF(64 * wv + point_lane(), PASS == DKDV ? a.Wi : a.Wo, PASS == DKDV ? a.Hi : a.Ho)
+    (void)c, (void)qd, (void)nvalid;
+    const int row = (PASS == DKDV ? a.sorder : a.gorder)[a.row_first + rowsel];
+    for (; redo; redo &= redo - 1) {
+        const int col = w0 + __builtin_ctz(redo);
+        if (PASS == FWD) point_forward<T, N>(a, b, h, bh, row, col, 0, a.dv_, true, lane);
+        if (PASS == DQ) point_dq<T, N>(a, b, h, bh, row, col, 0, a.dk_, true, lane);
+        if (PASS == DKDV) point_dkdv<T, N>(a, b, h, bh, row, col, 0, a.dk_, a.dv_, lane);
+    }
+}
+
 // ---- forward ---------------------------------------------------------------------------------------------------
 template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) void fwd_s16_kernel(const Args a)
 {
@@ -424,7 +439,11 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
     }
 
     Z = h16_quarter_sum(Z);
-    if (mine) {
+    float check = Z;
+#pragma unroll
+    for (int cb = 0; cb < NCB; cb++) check += point_sum(acc[cb].hi + acc[cb].lo);
+    const unsigned redo = point_columns(mine && not_finite(check));
+    if (mine && !(redo >> c & 1)) {
         if (a.lse && qd == 0) a.lse[((size_t)bh * a.Ho + ho) * a.Wo + w0 + c] = m + fast_log2(Z);
         const float inv = 1.0f / Z;
         T *y = static_cast<T *>(a.y) + pt * a.ldy + h * nv + 4 * qd;
@@ -432,6 +451,7 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
         for (int cb = 0; cb < NCB; cb++)
             if (!PAD || 16 * cb + 4 * qd < nv) s16_store4(y + 16 * cb, (acc[cb].hi + acc[cb].lo) * inv);
     }
+    if (redo) s16_points<T, NCB, FWD>(redo, wv);
 }
 
 // ---- backward, dq pass (needs the forward's y and lse) -------------------------------------------------------------
@@ -563,13 +583,18 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
     // (stored after the walk: a global store ahead of the loop would turn the loop's scalar loads of runs and weights,
     // which the compiler only uses while nothing in the kernel can have written memory, into vector loads with waits)
     off = EXACT_I ? 0.f : h16_quarter_sum(off);
-    if (mine && qd == 0) a.stats[sidx] = make_float2(lse, I + off);
-    if (mine) {
+    float check = off;
+#pragma unroll
+    for (int cb = 0; cb < NCB; cb++) check += point_sum(EXACT_I ? acc[cb].hi + acc[cb].lo : acc[cb].hi + acc[cb].lo + ak[EXACT_I ? 0 : cb]);
+    const unsigned redo = point_columns(mine && not_finite(check));
+    if (mine && !(redo >> c & 1)) {
+        if (qd == 0) a.stats[sidx] = make_float2(lse, I + off);
         T *dq = static_cast<T *>(a.dq) + pt * a.lddq + h * nk + 4 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++)
             if (!PAD || 16 * cb + 4 * qd < nk) s16_store4(dq + 16 * cb, EXACT_I ? acc[cb].hi + acc[cb].lo : (acc[cb].hi + acc[cb].lo) - off * ak[EXACT_I ? 0 : cb]);
     }
+    if (redo) s16_points<T, NCB, DQ>(redo, wv);
 }
 
 // ---- backward, dk/dv pass: transposed gather ---------------------------------------------------------------------
@@ -579,7 +604,7 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
 // fp32: q is staged times log2 e, rounded as the other two passes round it, so all three see the same scores (the gradients lean on
 // sums of dS that cancel exactly: q (k log2 e) instead doubles the noise in sum dk); dk takes the factor back at the end.  16-bit: q is
 // staged as it is, an exact term or two, and k carries the factor.
-template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW, D == 64 || (D == 48 && S16Piece<T>::S == 3) ? 2 : 3) void dkdv_s16_kernel(const Args a)
+template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW, D == 64 || (D == 48 && S16Piece<T>::S == 3) ? 2 : (D == 32 && S16Piece<T>::S == 1 ? 4 : 3)) void dkdv_s16_kernel(const Args a)
 {
     typedef SplitBand<T, D, PAD> Band_;
     constexpr int S = Band_::S, PITCH = Band_::PITCH, NCB = D / 16;
@@ -711,7 +736,11 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW, D =
         wk.advance();
     }
 
-    if (mine) {
+    float check = 0.f;
+#pragma unroll
+    for (int cb = 0; cb < NCB; cb++) check += point_sum(s16_value(dkt[cb]) + s16_value(dvt[cb]));
+    const unsigned redo = point_columns(mine && not_finite(check));
+    if (mine && !(redo >> c & 1)) {
         T *dk = static_cast<T *>(a.dk) + pt * a.lddk + h * nk + 4 * qd, *dv = static_cast<T *>(a.dv) + pt * a.lddv + h * nv + 4 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++) {
@@ -719,4 +748,5 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW, D =
             if (!PAD || 16 * cb + 4 * qd < nv) s16_store4(dv + 16 * cb, s16_value(dvt[cb]));
         }
     }
+    if (redo) s16_points<T, NCB, DKDV>(redo, wv);
 }
