@@ -34,8 +34,9 @@
  * no other.  Two kernel families give less: fp32 heads of 32 channels on large grids with mostly short runs, and 16-bit heads of equal
  * width (a multiple of 8, 16 to 256); there it may also reach points of the same batch entry and head whose neighborhoods share a tile
  * with the point: at most a tile (32 or 16 longitudes) and a run away in longitude, on the latitudes that see the point's latitude.  A
- * ring step may pass it to the 16 longitudes of a tile in the same way, and where its fp32 or fp16 operands are split an infinity counts as
- * NaN.  A quadrature weight of zero takes its latitude out of the softmax; y is NaN where nothing is left.
+ * ring step may pass it to the 16 longitudes of a tile in the same way, and where its fp32 or fp16 operands are split an infinity, and a
+ * magnitude above 3.38e38, counts as NaN.  Where fp32 operands are split (fp32 heads of up to 64 channels), magnitudes below 2^-110 are
+ * held to 2^-133 absolutely.  A quadrature weight of zero takes its latitude out of the softmax; y is NaN where nothing is left.
  */
 #ifndef S2ATTN_H
 #define S2ATTN_H
@@ -280,8 +281,10 @@ int s2attn_permute_to_nchw(const void *src, void *dst, int64_t B, int64_t H, int
  *   s2attn_grad_partials       partial sums over slices of the points of sum_n pm_p[n, j] cm[i, n] (weight gradients) and of both
  *                              operands alone (bias gradients)
  * Element type of the arithmetic (`compute`): S2ATTN_F32 takes fp32 tensors (products of three-term bf16 splits, fp32
- * accumulation: as exact as fp32 multiply-adds), S2ATTN_BF16 / S2ATTN_F16 16-bit ones, or an fp32 NCHW tensor that is rounded on
- * the way in (autocast) and its fp32 gradient.
+ * accumulation: as exact as fp32 multiply-adds for magnitudes from 2^-110 to 3.38e38), S2ATTN_BF16 / S2ATTN_F16 16-bit ones, or an fp32
+ * NCHW tensor that is rounded on the way in (autocast) and its fp32 gradient.  Below 2^-110 a value is held to 2^-133 absolutely (the
+ * third term of a split leaves bf16's range); above bf16's largest it counts as NaN.  A NaN or an infinity among the channels of a
+ * point makes its results NaN or infinite, not necessarily the infinity that exact arithmetic has; no other point's.
  *
  * Weights are packed once per call (s2attn_pack_weights) into blocks of 64 rows x 16 columns in the order the kernels take:
  * a job lays one matrix, element (r, c) at w[r * row_stride + c * col_stride], times scale, at rows 64 * first_block and

@@ -158,3 +158,42 @@ def test_what_is_not_finite_reaches_true_neighbors_only(shape, poison):
             assert_close(name, x, y, rtol=1e-5, atol=1e-5)
         else:
             assert_close(name, x, y, rtol=2e-2, atol=2e-2 * y.square().mean().sqrt().item())
+
+
+def _layer(dtype, channels, k_channels, out_channels, **kw):
+    from torch_harmonics_amd import NeighborhoodAttentionS2
+
+    torch.manual_seed(11)
+    m = NeighborhoodAttentionS2(channels, (10, 66), (10, 66), num_heads=2, k_channels=k_channels, out_channels=out_channels, theta_cutoff=0.5, **kw).cuda()
+    return m.to(dtype) if dtype != F32 else m
+
+
+@pytest.mark.parametrize("value", [NAN, INF, -3.4e38])
+@pytest.mark.parametrize("channels", [(17, 8, 40), (64, 40, 24)], ids=lambda c: f"c{c[0]}k{c[1]}o{c[2]}")
+def test_layer_keeps_what_is_not_finite_to_the_points_that_see_it(channels, value):
+    """The projections contract channels, never points, and the attention touches true neighbors: the layer's result is untouched
+    elsewhere, and not finite at every point whose neighborhood holds the value (an infinity may come out as NaN)."""
+    m = _layer(F32, *channels)
+    x = torch.randn(2, channels[0], 10, 66, device="cuda")
+    mask = oracle.dense_mask(m.psi_col_idx.cpu(), m.psi_roff_idx.cpu(), 10, 66, 10, 66).reshape(10, 66, 10, 66)[:, :, 4, 30].cuda()
+    for channel in (0, channels[0] - 1):
+        bad = x.clone()
+        bad[1, channel, 4, 30] = value
+        with torch.no_grad():
+            a, b = m(bad), m(x)
+        assert torch.equal(a[0], b[0])
+        assert not torch.isfinite(a[1][:, mask]).any() and torch.isfinite(a[1][:, ~mask]).all()
+        assert_close("elsewhere", a[1][:, ~mask], b[1][:, ~mask], rtol=1e-5, atol=1e-5)
+
+
+def test_small_magnitudes_keep_their_precision():
+    """Three bf16 terms hold a value to 2^-24 down to 2^-110, and to 2^-133 absolutely below: the layer is linear in its value input (three
+    products with sums of at most 40, 120 and 40 terms of magnitude below 4)."""
+    m = _layer(F32, 40, 40, 40, bias=False)
+    x, v = torch.randn(1, 40, 10, 66, device="cuda"), torch.randn(1, 40, 10, 66, device="cuda")
+    with torch.no_grad():
+        want = m(x, x, v).double()
+        for k in (60, 90, 105, 115, 120):
+            got = m(x, x, v * 2.0**-k).double() * 2.0**k
+            worst = ((got - want).abs() - 2.0**-22 * want.abs().max() - 200 * 2.0 ** (k - 133)).max().item()
+            assert worst <= 0, f"2^-{k}: {worst:.3e} beyond the bound"
