@@ -592,16 +592,11 @@ def main():
     d = k.shape[3] // nh
     # per launch: compulsory traffic (every tensor the kernel must read or write, once), algorithmic flops
     # (2*d per contraction per pair: forward q.k, p.v; dq pass q.k, dy.v, dq; dk/dv pass q.k, dy.v, dk, dv), time
-    if bf16:
-        kname = ("fwd_h16_kernel", "dq_h16_kernel", "dkdv_h16_kernel")
-    elif d == 64 or (d == 32 and min(Wi, Wo) < 64):
-        kname = ("fwd_s16_kernel", "dq_s16_kernel", "dkdv_s16_kernel")
-    elif d == 16:  # chosen by the size of the grid and the share of latitudes with long runs
-        kname = ("fwd_m32_kernel or fwd_s16_kernel", "dq_m32_kernel or dq_s16_kernel", "dkdv_m32_kernel or dkdv_s16_kernel")
-    elif d == 128:
-        kname = ("fwd_m32_kernel", "dq_m32_kernel", "dkdv_m32_kernel")
-    else:
-        kname = ("fwd_mfma_kernel", "dq_saved_mfma_kernel", "dkdv_mfma_kernel")
+    family = {"vector": "{}", "hybrid": "{}_mfma", "16bit": "{}_h16", "fp32": "{}_m32", "split": "{}_s16"}
+    kname = []
+    for i, name in enumerate(("fwd", "dq", "dkdv")):
+        f = _lib.FAMILIES[_lib.check(lib.s2attn_attention_family(i, pl, sh, 16), "family")]
+        kname.append(family[f].format("dq_saved" if f == "hybrid" and name == "dq" else name) + "_kernel")
     alg = {
         f"s2::{kname[0]} (forward)": (esz * (nq + nk + nv + ny) + 4 * nstat, 4 * d * pairs, t_fwd),
         f"s2::{kname[1]} (backward, dq)": (esz * (nq + nk + nv + ny + ny + nq) + 12 * nstat, 6 * d * pairs, t_dq),

@@ -197,6 +197,17 @@ int s2attn_forward_lse(const void *k, const void *v, const void *q, const float 
                        const s2attn_plan *plan, const s2attn_shape *shape, void *stream);
 
 /*
+ * The family of kernels that a pass (0 forward, 1 dq from saved statistics, 2 dk/dv) of this problem runs on when every tensor's
+ * address is a multiple of `alignment` bytes, or a negative error.  Host only: nothing is launched or read on the device.
+ */
+#define S2ATTN_FAMILY_VECTOR 0 /* neighbor by neighbor */
+#define S2ATTN_FAMILY_HYBRID 1 /* fp32 heads of 32 channels: long runs on fp32 matrix instructions, short ones neighbor by neighbor */
+#define S2ATTN_FAMILY_16BIT 2  /* 16-bit matrix instructions */
+#define S2ATTN_FAMILY_FP32 3   /* fp32 matrix instructions, 16 longitudes per wavefront */
+#define S2ATTN_FAMILY_SPLIT 4  /* fp32 accuracy on bf16 matrix instructions, operands split into bf16 terms */
+int s2attn_attention_family(int pass, const s2attn_plan *plan, const s2attn_shape *shape, int alignment);
+
+/*
  * Backward.  Replaces attention_kernels::backward (attention_interface.cpp:117-119;
  * CUDA implementation s2_attention_bwd_dkvq_cuda, attention_cuda_bwd.cu:856-956).
  * Writes dk, dv, dq (every element; no pre-zeroing needed, no atomics).

@@ -10,46 +10,56 @@ import torch
 
 from oracle import cpu_attention as oracle
 from oracle import geometry as ogeo
+from tests.families import families
 from tests.test_gpu_widths import BF16, F16, F32, _bounds
 from tests.util import assert_close, randn_inputs
 
 pytestmark = pytest.mark.gpu
 
-# storage, ck, cv, grid (one, or input and output grid), batch copies, heads.  Copies of one batch entry: the fp32 dispatch goes by the
+# storage, ck, cv, grid (one, or input and output grid), batch copies, heads, family of kernels of all three passes.  Copies of one batch entry: the fp32 dispatch goes by the
 # number of workgroups (heads of up to 16 channels: 1024, heads of 32: 4096), the oracle by one entry.
 SHAPES = {
-    "f32_c3c5": (F32, 3, 5, (9, 48), 1, 2),  # vector kernels
-    "f32_c8": (F32, 8, 8, (9, 48), 1, 2),  # 16-longitude fp32 tiles, few workgroups
-    "f32_c8_many": (F32, 8, 8, (9, 48), 60, 2),  # split products
-    "f32_c4c12_many": (F32, 4, 12, (9, 48), 60, 2),
-    "f32_c16_many": (F32, 16, 16, (9, 48), 60, 2),
-    "f32_c20c12": (F32, 20, 12, (9, 48), 1, 2),
-    "f32_c20c12_down": (F32, 20, 12, ((9, 96), (5, 48)), 1, 2),
-    "f32_c20c12_up": (F32, 20, 12, ((5, 34), (9, 102)), 1, 2),
-    "f32_c32": (F32, 32, 32, (9, 64), 1, 2),
-    "f32_c32_many": (F32, 32, 32, (16, 64), 128, 2),  # hybrid kernels over short runs
-    "f32_c40": (F32, 40, 40, (9, 48), 1, 2),
-    "f32_c64": (F32, 64, 64, (9, 48), 1, 2),
-    "f32_c68c20": (F32, 68, 20, (9, 48), 1, 2),  # fp32 tiles of 128 channels
-    "f32_c68c20_down": (F32, 68, 20, ((9, 96), (5, 48)), 1, 2),
-    "f32_c68c20_up": (F32, 68, 20, ((5, 34), (9, 102)), 1, 2),
-    "f32_c160": (F32, 160, 160, (9, 48), 1, 1),  # two channel groups
-    "f32_c20c132": (F32, 20, 132, (9, 48), 1, 1),
-    "bf16_c32": (BF16, 32, 32, (9, 48), 1, 2),  # 16-bit tiles
-    "bf16_c20c12": (BF16, 20, 12, (9, 48), 1, 2),  # split products
-    "bf16_c12": (BF16, 12, 12, (9, 48), 1, 2),
-    "f16_c64": (F16, 64, 64, (9, 48), 1, 2),
-    "f16_c36c44": (F16, 36, 44, (9, 48), 1, 2),
-    "f16_c36c44_up": (F16, 36, 44, ((5, 34), (9, 102)), 1, 2),
+    "f32_c3c5": (F32, 3, 5, (9, 48), 1, 2, "vector"),
+    "f32_c8": (F32, 8, 8, (9, 48), 1, 2, "fp32"),
+    "f32_c8_many": (F32, 8, 8, (9, 48), 60, 2, "split"),
+    "f32_c4c12_many": (F32, 4, 12, (9, 48), 60, 2, "split"),
+    "f32_c16_many": (F32, 16, 16, (9, 48), 60, 2, "split"),
+    "f32_c20c12": (F32, 20, 12, (9, 48), 1, 2, "split"),
+    "f32_c20c12_down": (F32, 20, 12, ((9, 96), (5, 48)), 1, 2, "split"),
+    "f32_c20c12_up": (F32, 20, 12, ((5, 34), (9, 102)), 1, 2, "split"),
+    "f32_c32": (F32, 32, 32, (9, 64), 1, 2, "split"),
+    "f32_c32_many": (F32, 32, 32, (16, 64), 128, 2, "hybrid"),
+    "f32_c40": (F32, 40, 40, (9, 48), 1, 2, "split"),
+    "f32_c64": (F32, 64, 64, (9, 48), 1, 2, "split"),
+    "f32_c68c20": (F32, 68, 20, (9, 48), 1, 2, "fp32"),
+    "f32_c68c20_down": (F32, 68, 20, ((9, 96), (5, 48)), 1, 2, "fp32"),
+    "f32_c68c20_up": (F32, 68, 20, ((5, 34), (9, 102)), 1, 2, "fp32"),
+    "f32_c160": (F32, 160, 160, (9, 48), 1, 1, "fp32"),  # two channel groups
+    "f32_c20c132": (F32, 20, 132, (9, 48), 1, 1, "fp32"),
+    "bf16_c32": (BF16, 32, 32, (9, 48), 1, 2, "16bit"),
+    "bf16_c20c12": (BF16, 20, 12, (9, 48), 1, 2, "split"),
+    "bf16_c12": (BF16, 12, 12, (9, 48), 1, 2, "split"),
+    "f16_c64": (F16, 64, 64, (9, 48), 1, 2, "16bit"),
+    "f16_c36c44": (F16, 36, 44, (9, 48), 1, 2, "split"),
+    "f16_c36c44_up": (F16, 36, 44, ((5, 34), (9, 102)), 1, 2, "split"),
 }
 TILES = {"f32_c32_many", "bf16_c32", "f16_c64"}  # what is not finite may reach the columns of a whole tile
 
 
+def _theta(shape, fine, coarse):
+    """Disk radius for the shape's input grid; the hybrid kernels take mostly short runs."""
+    grid = SHAPES[shape][3]
+    if SHAPES[shape][6] == "hybrid":
+        return 0.3
+    return coarse if isinstance(grid[0], tuple) and grid[0][0] == 5 else fine
+
+
 def _problem(shape, theta):
-    dtype, ck, cv, grid, copies, nh = SHAPES[shape]
+    dtype, ck, cv, grid, copies, nh, family = SHAPES[shape]
     ins, outs = grid if isinstance(grid[0], tuple) else (grid, grid)
     up = oracle.is_upsample(ins[1], outs[1])
     col, roff = ogeo.neighborhood_csr(*((outs, ins) if up else (ins, outs)), "equiangular", "equiangular", theta)
+    assert set(families(dtype, copies, nh, ck, cv, ins, outs, col, roff)) == {family}
     quad = ogeo.attention_quad_weights(*ins, "equiangular")
     mask = (oracle.dense_mask_upsample if up else oracle.dense_mask)(col, roff, *ins, *outs)
     tensors = [t.to(dtype) for t in randn_inputs(1, *ins, *outs, nh, ck, cv, scale=1.0 if dtype == F32 else 0.5)]
@@ -96,7 +106,9 @@ def _true_neighbors(tensors, quad, mask, nh):
 def test_quadrature_weight_zero(shape, zero):
     """A latitude of quadrature weight zero takes no part in the softmax, wherever it stands in a query's neighborhood (the reference
     multiplies by the weight, attention_torch.py:97-125).  all_but_one: with a disk that holds the whole sphere."""
-    dtype, tensors, quad, geometry, mask = _problem(shape, 4.0 if zero == "all_but_one" else 0.9 if SHAPES[shape][3][0] in (9, 16) or isinstance(SHAPES[shape][3][0], tuple) and SHAPES[shape][3][0][0] == 9 else 1.7)
+    if zero in ("first_two", "all_but_one") and SHAPES[shape][6] == "hybrid":
+        pytest.skip("needs a disk of a radius that has long runs only")
+    dtype, tensors, quad, geometry, mask = _problem(shape, 4.0 if zero == "all_but_one" else _theta(shape, 0.9, 1.7))
     H = quad.numel()
     quad = quad.clone()
     quad[{"first": slice(0, 1), "middle": slice(H // 2, H // 2 + 1), "first_two": slice(0, 2), "all_but_one": slice(0, H - 2)}[zero]] = 0.0
@@ -127,7 +139,7 @@ POISON = {"k_nan": (0, NAN), "v_nan": (1, NAN), "q_nan": (2, NAN), "dy_nan": (3,
 def test_what_is_not_finite_reaches_true_neighbors_only(shape, poison):
     """One channel of one point is NaN, infinite or of a magnitude that only fp32 holds: what sees the point gets what float64
     arithmetic on its neighbors gives, and everything else the result it has without it."""
-    dtype, tensors, quad, geometry, mask = _problem(shape, 0.6 if SHAPES[shape][3][0] in (9, 16) or isinstance(SHAPES[shape][3][0], tuple) and SHAPES[shape][3][0][0] == 9 else 0.9)
+    dtype, tensors, quad, geometry, mask = _problem(shape, _theta(shape, 0.6, 0.9))
     if poison == "weight_below_zero":
         quad = quad.clone()
         quad[quad.numel() // 2] *= -0.01  # (the sums must not cancel)

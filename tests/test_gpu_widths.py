@@ -14,6 +14,7 @@ import torch
 
 from oracle import cpu_attention as oracle
 from oracle import geometry as ogeo
+from tests.families import families
 from tests.util import assert_close, randn_inputs
 
 pytestmark = pytest.mark.gpu
@@ -76,3 +77,78 @@ def test_head_widths(widths, grid, dtype):
             assert torch.isfinite(got).all() and worst <= 0, f"{name}: {worst:.3e} beyond the bound"
     for a, b in zip(grads, plain):  # the backward that recomputes y and its normaliser runs the same kernels on them
         assert torch.equal(a, b)
+
+
+# fp32 heads of up to 16 channels: which kernels run goes by the number of workgroups (1024, and for dk/dv over short runs 4096) and by
+# the share of latitudes with long runs.  widths, grid, theta, batch, families of the three passes
+NARROW = [
+    ((4, 4), (7, 32), 0.5, 60, ("fp32", "split", "split")),
+    ((4, 4), (7, 32), 1.2, 60, ("split", "split", "split")),
+    ((8, 12), (6, 33), 2.0, 60, ("split", "split", "split")),
+    ((16, 16), (9, 79), 0.45, 30, ("split", "split", "split")),
+    ((12, 16), (5, 80), 4.0, 60, ("split", "split", "split")),
+    ((16, 4), (8, 130), 0.3, 20, ("split", "split", "split")),
+    ((16, 16), (16, 64), 0.2, 30, ("fp32", "split", "split")),
+    ((8, 8), (16, 64), 0.2, 90, ("fp32", "split", "fp32")),
+    ((4, 12), (16, 64), 0.2, 30, ("fp32", "split", "split")),
+    ((16, 16), (16, 64), 0.2, 1, ("fp32", "fp32", "fp32")),
+]
+
+
+def _against_float64(results, k, v, q, dy, quad, col, roff, nh):
+    kr, vr, qr = [t.double().requires_grad_(True) for t in (k, v, q)]
+    y = oracle.dense_attention_f64(kr, vr, qr, quad, col, roff, nh)
+    y.backward(dy.double())
+    for name, got, want in zip(("y", "dk", "dv", "dq"), results, (y.detach(), kr.grad, vr.grad, qr.grad)):
+        assert_close(name, got, want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("case", NARROW, ids=lambda c: f"ck{c[0][0]}cv{c[0][1]}_{c[1][0]}x{c[1][1]}_{c[2]}_b{c[3]}")
+def test_narrow_fp32_heads_on_every_family(case):
+    from torch_harmonics_amd import ops
+
+    (ck, cv), grid, theta, batch, want = case
+    nh = 3
+    col, roff = ogeo.neighborhood_csr(grid, grid, "equiangular", "equiangular", theta)
+    assert families(F32, batch, nh, ck, cv, grid, grid, col, roff) == want
+    quad = ogeo.attention_quad_weights(*grid, "equiangular")
+    tensors = randn_inputs(2, *grid, *grid, nh, ck, cv)
+    kd, vd, qd, gd = [t.cuda()[torch.arange(batch) % 2] for t in tensors]  # two entries, repeated
+    geo = (quad.cuda(), col.cuda(), roff.cuda(), nh, grid[1], *grid)
+    y, lse = ops.forward_lse(kd, vd, qd, *geo)
+    results = [y, *ops.backward_saved(kd, vd, qd, gd, y, lse, *geo)]
+    for t in results:
+        for i in range(2):
+            assert torch.equal(t[i::2], t[i : i + 1].expand(t[i::2].shape)) if i < batch else True
+    if batch > 1:
+        _against_float64([t[:2] for t in results], *tensors, quad, col, roff, nh)
+    else:
+        _against_float64(results, *[t[:1] for t in tensors], quad, col, roff, nh)
+
+
+@pytest.mark.parametrize("offset", [1, 2])
+@pytest.mark.parametrize("widths", [(4, 4), (8, 8), (16, 12), (20, 12), (32, 32), (48, 48), (64, 64), (68, 20)], ids=lambda w: f"ck{w[0]}cv{w[1]}")
+def test_fp32_tensors_at_any_element(widths, offset):
+    """Tensors that start at any multiple of four bytes: the split products take them as they are (up to 64 channels), wider heads go to
+    the vector kernels."""
+    from torch_harmonics_amd import ops
+
+    (ck, cv), grid, nh = widths, (9, 66), 2
+    col, roff = ogeo.neighborhood_csr(grid, grid, "equiangular", "equiangular", 0.5)
+    assert set(families(F32, 1, nh, ck, cv, grid, grid, col, roff, alignment=4 * offset)) == {"split" if ck <= 64 else "vector"}
+    quad = ogeo.attention_quad_weights(*grid, "equiangular")
+    tensors = randn_inputs(1, *grid, *grid, nh, ck, cv)
+
+    def shifted(t):
+        room = torch.empty(t.numel() + offset, device="cuda")
+        room[offset:] = t.flatten()
+        return room[offset:].view(t.shape)
+
+    kd, vd, qd, gd = [shifted(t) for t in tensors]
+    assert all(t.is_contiguous() and t.data_ptr() % 16 == 4 * offset for t in (kd, vd, qd, gd))
+    geo = (quad.cuda(), col.cuda(), roff.cuda(), nh, grid[1], *grid)
+    y, lse = ops.forward_lse(kd, vd, qd, *geo)
+    results = [y, *ops.backward_saved(kd, vd, qd, gd, y, lse, *geo)]
+    _against_float64(results, *tensors, quad, col, roff, nh)
+    for a, b in zip(results[1:], ops.backward(kd, vd, qd, gd, *geo)):
+        assert_close("recomputed", a, b, rtol=1e-5, atol=1e-5)

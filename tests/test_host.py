@@ -14,6 +14,7 @@ import torch
 
 import torch_harmonics_amd as tha
 from oracle import geometry as ogeo
+from tests.families import families
 from torch_harmonics_amd import _lib, ops
 from torch_harmonics_amd.neighborhood import precompute_neighborhood_s2
 from torch_harmonics_amd.plan import build_host_plan
@@ -794,3 +795,30 @@ def test_module_constructor_time_at_the_headline_grid():
     dt = time.perf_counter() - t0
     print(f"constructor at 721x1440: {dt * 1e3:.0f} ms")
     assert m.psi_col_idx.numel() == 99625 and dt < 1.0
+
+
+# ---- dispatch --------------------------------------------------------------------------------------
+F32, BF16, F16 = torch.float32, torch.bfloat16, torch.float16
+FAMILY_CASES = [
+    # dtype, ck, cv, grid, batch, alignment, family of the forward
+    (F32, 64, 64, (12, 64), 1, 16, "split"), (F32, 64, 64, (12, 64), 1, 4, "split"), (F32, 64, 64, (12, 31), 1, 16, "vector"), (F32, 63, 63, (12, 64), 1, 16, "vector"),
+    (F32, 68, 64, (12, 64), 1, 16, "fp32"), (F32, 68, 64, (12, 64), 1, 8, "vector"), (F32, 512, 512, (12, 64), 1, 16, "fp32"), (F32, 32, 32, (12, 64), 1, 16, "split"),
+    (F32, 16, 16, (12, 64), 1, 16, "fp32"), (F32, 16, 16, (12, 64), 1, 8, "split"), (F32, 16, 16, (12, 64), 128, 16, "split"),
+    (BF16, 32, 32, (12, 64), 1, 16, "16bit"), (BF16, 32, 32, (12, 64), 1, 8, "split"), (BF16, 32, 32, (12, 64), 1, 4, "vector"), (BF16, 20, 20, (12, 64), 1, 8, "split"),
+    (F16, 256, 256, (12, 64), 1, 16, "16bit"), (F16, 264, 264, (12, 64), 1, 16, "vector"), (F16, 68, 60, (12, 64), 1, 16, "vector"), (F16, 8, 8, (12, 64), 1, 16, "split"),
+]  # fmt: skip
+
+
+@pytest.mark.parametrize("case", FAMILY_CASES, ids=lambda c: f"{str(c[0])[6:]}_ck{c[1]}cv{c[2]}_w{c[3][1]}_b{c[4]}_a{c[5]}")
+def test_family_of_kernels(case):
+    dtype, ck, cv, grid, batch, alignment, want = case
+    col, roff = ogeo.neighborhood_csr(grid, grid, "equiangular", "equiangular", 0.9)
+    assert families(dtype, batch, 2, ck, cv, grid, grid, col, roff, alignment)[0] == want
+
+
+def test_family_of_kernels_checks_its_arguments():
+    col, roff = ogeo.neighborhood_csr((6, 12), (6, 12), "equiangular", "equiangular", 0.9)
+    with pytest.raises(RuntimeError, match="alignment"):
+        families(F32, 1, 1, 4, 4, (6, 12), (6, 12), col, roff, alignment=0)
+    with pytest.raises(RuntimeError, match="positive"):
+        families(F32, 0, 1, 4, 4, (6, 12), (6, 12), col, roff)

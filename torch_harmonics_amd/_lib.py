@@ -121,6 +121,9 @@ class RingUpShapeStruct(ctypes.Structure):
     ]
 
 
+# s2attn_attention_family: the names of the families
+FAMILIES = ("vector", "hybrid", "16bit", "fp32", "split")
+
 # every symbol include/s2attn.h declares: name -> (restype, argtypes)
 SYMBOLS = {
     "s2attn_last_error": (ctypes.c_char_p, []),
@@ -130,6 +133,7 @@ SYMBOLS = {
     "s2attn_plan_build": (_int, [_vp, _vp, _i64, _int, _int, _int, _int, _vp, _i64]),
     "s2attn_forward": (_int, [_vp, _vp, _vp, _vp, _vp, ctypes.POINTER(PlanStruct), ctypes.POINTER(ShapeStruct), _vp]),
     "s2attn_forward_lse": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, ctypes.POINTER(PlanStruct), ctypes.POINTER(ShapeStruct), _vp]),
+    "s2attn_attention_family": (_int, [_int, ctypes.POINTER(PlanStruct), ctypes.POINTER(ShapeStruct), _int]),
     "s2attn_backward_saved": (_int, [_vp] * 11 + [ctypes.POINTER(PlanStruct), ctypes.POINTER(ShapeStruct), _vp]),
     "s2attn_backward_saved_noalloc": (_int, [_vp] * 10 + [ctypes.POINTER(PlanStruct), ctypes.POINTER(ShapeStruct), _vp]),
     "s2attn_backward_dq_saved": (_int, [_vp] * 9 + [ctypes.POINTER(PlanStruct), ctypes.POINTER(ShapeStruct), _vp]),
@@ -231,8 +235,9 @@ def load_torch_ops() -> None:
         _torch_ops_loaded = True
 
 
-def check(rc: int, what: str) -> None:
-    """Turns a negative return code into a RuntimeError carrying the library's message."""
+def check(rc: int, what: str) -> int:
+    """Turns a negative return code into a RuntimeError carrying the library's message; returns any other."""
     if rc < 0:
         msg = load().s2attn_last_error()
         raise RuntimeError(f"{what}: {msg.decode() if msg else f'error {rc}'}")
+    return rc

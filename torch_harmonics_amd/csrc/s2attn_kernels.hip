@@ -2789,54 +2789,62 @@ bool dense_ok(Which which, const Args &a, bool vec)
     return vec && a.dk_ == 32 && a.dv_ == 32 && a.Wi >= 64;
 }
 
+// The family of kernels that takes a problem
+template <typename T> int family_t(Which which, const Args &a, bool vec, int ndense)
+{
+    const bool hybrid = dense_ok(which, a, vec);
+    if constexpr (std::is_same<T, float>::value) {
+        const bool other = hybrid || (std::max(a.dk_, a.dv_) <= 16 && m32_ok<T>(which, a));
+        if (s16_ok<T>(which, a) && (s16_faster(which, a, ndense) || !other)) return S2ATTN_FAMILY_SPLIT;
+    }
+    if (a.unpacked) return S2ATTN_FAMILY_HYBRID;
+    if (h16_ok<T>(which, a)) return S2ATTN_FAMILY_16BIT;
+    if (!std::is_same<T, float>::value && s16_ok<T>(which, a)) return S2ATTN_FAMILY_SPLIT;
+    // head dim 32 on at least 64 columns: the hybrid kernels handle short runs themselves (vector path inside), so
+    // they take every latitude; measured ahead of the 16-longitude family there (cfg3 13.5 against 16.4 ms)
+    if (hybrid) return S2ATTN_FAMILY_HYBRID;
+    return m32_ok<T>(which, a) ? S2ATTN_FAMILY_FP32 : S2ATTN_FAMILY_VECTOR;
+}
+
 template <typename T> int launch_t(Which which, const Args &a, bool vec, int ndense, hipStream_t stream)
 {
-    const int nrows = which == DKDV ? a.Hi : a.Ho;
-    int first = 0;
     // column blocks of a wider buffer: only the hybrid and the split kernels address every tensor by its own point stride, and
     // callers rely on the former's domain
     if (a.unpacked && !dense_ok(which, a, vec))
         return s2attn_fail(S2ATTN_E_UNSUPPORTED, "tensors with a point stride need the hybrid kernels: ck = cv = 32, 16-byte aligned, at least 64 longitudes%s",
                            which == DQ ? ", backward from saved statistics" : "");
     const int d = std::max(a.dk_, a.dv_);
-    if constexpr (std::is_same<T, float>::value) {
-        if (s16_ok<T>(which, a) && (s16_faster(which, a, ndense) || !(dense_ok(which, a, vec) || (d <= 16 && m32_ok<T>(which, a))))) {
+    switch (family_t<T>(which, a, vec, ndense)) {
+    case S2ATTN_FAMILY_SPLIT:
+        if constexpr (std::is_same<T, float>::value) {
             const bool exact = a.dk_ == a.dv_;
-            if (d <= 16) return exact && d == 16 ? launch_s16<T, 16, false>(which, a, stream) : launch_s16<T, 16, true>(which, a, stream);
-            if (d <= 32) return exact && d == 32 ? launch_s16<T, 32, false>(which, a, stream) : launch_s16<T, 32, true>(which, a, stream);
-            if (d <= 48) return launch_s16<T, 48, true>(which, a, stream);
-            return exact && d == 64 ? launch_s16<T, 64, false>(which, a, stream) : launch_s16<T, 64, true>(which, a, stream);
+            if (d == 16 && exact) return launch_s16<T, 16, false>(which, a, stream);
+            if (d == 32 && exact) return launch_s16<T, 32, false>(which, a, stream);
+            if (d == 64 && exact) return launch_s16<T, 64, false>(which, a, stream);
         }
-    }
-    if (a.unpacked) return launch_dense<T>(which, a, stream);
-    if (h16_ok<T>(which, a)) {
-        if (a.dk_ == 32) return launch_h16<T, 32, false>(which, a, stream);
-        if (a.dk_ == 64) return launch_h16<T, 64, false>(which, a, stream);
-        if (a.dk_ == 128) return launch_h16<T, 128, false>(which, a, stream);
-        if (a.dk_ < 32) return launch_h16<T, 32, true>(which, a, stream);
-        if (a.dk_ < 64) return launch_h16<T, 64, true>(which, a, stream);
-        if (a.dk_ < 128) return launch_h16<T, 128, true>(which, a, stream);
-        return launch_h16<T, 256, true>(which, a, stream);
-    }
-    if constexpr (!std::is_same<T, float>::value) {
-        if (s16_ok<T>(which, a)) {
-            if (d <= 16) return launch_s16<T, 16, true>(which, a, stream);
-            if (d <= 32) return launch_s16<T, 32, true>(which, a, stream);
-            return d <= 48 ? launch_s16<T, 48, true>(which, a, stream) : launch_s16<T, 64, true>(which, a, stream);
+        if (d <= 16) return launch_s16<T, 16, true>(which, a, stream);
+        if (d <= 32) return launch_s16<T, 32, true>(which, a, stream);
+        return d <= 48 ? launch_s16<T, 48, true>(which, a, stream) : launch_s16<T, 64, true>(which, a, stream);
+    case S2ATTN_FAMILY_HYBRID: return launch_dense<T>(which, a, stream);
+    case S2ATTN_FAMILY_16BIT:
+        if constexpr (!std::is_same<T, float>::value) {
+            if (a.dk_ == 32) return launch_h16<T, 32, false>(which, a, stream);
+            if (a.dk_ == 64) return launch_h16<T, 64, false>(which, a, stream);
+            if (a.dk_ == 128) return launch_h16<T, 128, false>(which, a, stream);
+            if (a.dk_ < 32) return launch_h16<T, 32, true>(which, a, stream);
+            if (a.dk_ < 64) return launch_h16<T, 64, true>(which, a, stream);
+            if (a.dk_ < 128) return launch_h16<T, 128, true>(which, a, stream);
+            return launch_h16<T, 256, true>(which, a, stream);
         }
-    }
-    if (dense_ok(which, a, vec)) {
-        // head dim 32 on at least 64 columns: the hybrid kernels handle short runs themselves (vector path inside), so
-        // they take every latitude; measured ahead of the 16-longitude family there (cfg3 13.5 against 16.4 ms)
-        return launch_dense<T>(which, a, stream);
-    }
-    if (m32_ok<T>(which, a)) {
+        break;
+    case S2ATTN_FAMILY_FP32:
         if (d <= 16) return launch_m32<16, 1>(which, a, stream);
         if (d <= 128) return launch_m32<128, 1>(which, a, stream);
         if (d <= 256) return launch_m32<128, 2>(which, a, stream);
         return d <= 384 ? launch_m32<128, 3>(which, a, stream) : launch_m32<128, 4>(which, a, stream);
     }
-    return vec ? launch_p<T, true>(which, a, first, nrows - first, stream) : launch_p<T, false>(which, a, first, nrows - first, stream);
+    const int nrows = which == DKDV ? a.Hi : a.Ho;
+    return vec ? launch_p<T, true>(which, a, 0, nrows, stream) : launch_p<T, false>(which, a, 0, nrows, stream);
 }
 
 int launch(Which which, const Args &a, int dtype, bool vec, int ndense, hipStream_t stream)
@@ -2902,6 +2910,24 @@ void fill_args(Args &a, const s2attn_plan *plan, const s2attn_shape *sh, const f
 
 
 } // namespace
+
+extern "C" int s2attn_attention_family(int pass, const s2attn_plan *plan, const s2attn_shape *shape, int alignment)
+{
+    int rc = check_shape(shape);
+    if (rc != S2ATTN_OK) return rc;
+    rc = check_plan(plan, shape);
+    if (rc != S2ATTN_OK) return rc;
+    if (pass < FWD || pass > DKDV || alignment < 1) return s2attn_fail(S2ATTN_E_INVALID, "pass is 0, 1 or 2, the alignment at least 1");
+    Args a = {};
+    fill_args(a, plan, shape, nullptr);
+    void *const at = reinterpret_cast<void *>((uintptr_t)alignment); // only its alignment is looked at
+    a.k = a.v = a.q = a.dy = a.ysaved = at, a.y = a.dk = a.dv = a.dq = at, a.lse = static_cast<float *>(at);
+    const bool vec = shape->ck % 4 == 0 && shape->cv % 4 == 0 && aligned(at, 4 * (size_t)esize(shape->dtype));
+    const Which which = static_cast<Which>(pass);
+    const int ndense = plan->header[which == DKDV ? S2ATTN_PH_SCATTER_NDENSE : S2ATTN_PH_GATHER_NDENSE];
+    if (shape->dtype == S2ATTN_F32) return family_t<float>(which, a, vec, ndense);
+    return shape->dtype == S2ATTN_BF16 ? family_t<bf16_t>(which, a, vec, ndense) : family_t<f16_t>(which, a, vec, ndense);
+}
 
 extern "C" int s2attn_forward_lse(const void *k, const void *v, const void *q, const float *quad_weights, void *y, float *lse,
                                   const s2attn_plan *plan, const s2attn_shape *shape, void *stream);
