@@ -31,12 +31,12 @@
  * elements of dq (wide heads) and dk (sums over many queries of both signs) up to 0.2 RMS off in a sweep of random problems.
  *
  * Values that are not finite: a NaN or an infinity reaches the points that see it, as arithmetic on each point's neighbors has it, and
- * no other.  Two kernel families give less: fp32 heads of 32 channels on large grids with mostly short runs, and 16-bit heads of equal
- * width (a multiple of 8, 16 to 256); there it may also reach points of the same batch entry and head whose neighborhoods share a tile
- * with the point: at most a tile (32 or 16 longitudes) and a run away in longitude, on the latitudes that see the point's latitude.  A
- * ring step may pass it to the 16 longitudes of a tile in the same way, and where its fp32 or fp16 operands are split an infinity, and a
- * magnitude above 3.38e38, counts as NaN.  Where fp32 operands are split (fp32 heads of up to 64 channels), magnitudes below 2^-110 are
- * held to 2^-133 absolutely.  A quadrature weight of zero takes its latitude out of the softmax; y is NaN where nothing is left.
+ * no other.  Fp32 heads of 32 channels and 16-bit heads of equal width (a multiple of 8, 16 to 256) give less: there it may also reach
+ * points of the same batch entry and head whose neighborhoods share a tile with the point: at most a tile (32 or 16 longitudes) and a
+ * run away in longitude, on the latitudes that see the point's latitude; what stays finite has the bits it has without it.  A ring step
+ * may pass it to the 16 longitudes of a tile in the same way, and where its fp32 or fp16 operands are split an infinity, and a magnitude
+ * above 3.38e38, counts as NaN.  Where fp32 operands are split (fp32 heads of up to 64 channels), magnitudes below 2^-110 are held to
+ * 2^-133 absolutely.  A quadrature weight of zero takes its latitude out of the softmax; y is NaN where nothing is left.
  */
 #ifndef S2ATTN_H
 #define S2ATTN_H

@@ -43,7 +43,7 @@ SHAPES = {
     "f16_c36c44": (F16, 36, 44, (9, 48), 1, 2, "split"),
     "f16_c36c44_up": (F16, 36, 44, ((5, 34), (9, 102)), 1, 2, "split"),
 }
-TILES = {"f32_c32_many", "bf16_c32", "f16_c64"}  # what is not finite may reach the columns of a whole tile
+TILES = {"f32_c32", "f32_c32_many", "bf16_c32", "f16_c64"}  # what is not finite may reach the columns of a whole tile
 
 
 def _theta(shape, fine, coarse):
@@ -128,6 +128,27 @@ def test_quadrature_weight_zero(shape, zero):
     for name, a, b, bound in zip(("y", "dk", "dv", "dq"), got, want, _bounds(k, v, q, dy, quad, mask, geometry[2], 2.0**-8 if dtype == BF16 else 2.0**-11)):
         worst = ((a.double() - b).abs() - bound).max().item()
         assert torch.isfinite(a).all() and worst <= 0, f"{name}: {worst:.3e} beyond the bound"
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38])
+def test_heads_of_32_channels_keep_an_infinity_where_it_is_seen(value):
+    """Split products of heads of 32 channels: a query that sees the value gets what arithmetic on its neighbors gives; what stays finite
+    has the bits it has without the value."""
+    dtype, tensors, quad, geometry, mask = _problem("f32_c32", 0.6)
+    clean = _run(tensors, quad, geometry)[0]
+    H, W = tensors[1].shape[1:3]
+    tensors[1][0, H // 2, W // 3, 1] = value
+    got, want = _run(tensors, quad, geometry)[0], _true_neighbors(tensors, quad, mask, geometry[2])[0]
+    sees = mask[:, (H // 2) * W + W // 3].reshape(1, H, W)
+    a, b = got[sees].double(), want[sees]
+    special = torch.isnan(b) | torch.isinf(b)
+    assert torch.equal(torch.isfinite(a), ~special)
+    assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(a[torch.isinf(b)], b[torch.isinf(b)])
+    big = b.abs() > 1e30
+    assert_close("seen", a[~special & ~big], b[~special & ~big], rtol=1e-5, atol=1e-5)
+    assert_close("seen, near the end of the range", a[~special & big] / 1e38, b[~special & big] / 1e38, rtol=1e-5, atol=0)
+    unseen = got[~sees]
+    assert torch.equal(unseen[torch.isfinite(unseen)], clean[~sees][torch.isfinite(unseen)])
 
 
 NAN, INF = float("nan"), float("inf")

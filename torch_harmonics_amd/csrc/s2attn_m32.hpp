@@ -176,18 +176,19 @@ template <typename T> __device__ inline u4v m32_piece(const char *p)
     return u4v{__float_as_uint(x.x), __float_as_uint(x.y), __float_as_uint(x.z), __float_as_uint(x.w)};
 }
 
-// The columns `redo` of a wavefront whose sums are not finite: its own channel group of them (see s2attn_points.hpp)
+// The columns `redo` of a wavefront whose sums are not finite, stored already: its own channel group of them (see s2attn_points.hpp)
 template <int D, int NS, Which PASS> __device__ inline void m32_points(unsigned redo)
 {
+    __threadfence(); // what is written here comes after it
     const Args a = point_args();
     S2_M32_IDS_OF(point_lane(), PASS == DKDV ? a.Wi : a.Wo, PASS == DKDV ? a.Hi : a.Ho)
     (void)c, (void)qd, (void)nvalid, (void)ldbk_, (void)ldbv_;
     const int row = (PASS == DKDV ? a.sorder : a.gorder)[a.row_first + rowsel];
     for (; redo; redo &= redo - 1) {
         const int col = w0 + __builtin_ctz(redo);
-        if (PASS == FWD) point_forward<float, D / 16>(a, b, h, bh, row, col, cbase, nv, wv == 0, lane);
-        if (PASS == DQ) point_dq<float, D / 16>(a, b, h, bh, row, col, cbase, nk, false, lane);
-        if (PASS == DKDV) point_dkdv<float, D / 16>(a, b, h, bh, row, col, cbase, nk, nv, lane);
+        if (PASS == FWD) point_forward<float, D / 16, false>(a, b, h, bh, row, col, cbase, nv, wv == 0, lane);
+        if (PASS == DQ) point_dq<float, D / 16, false>(a, b, h, bh, row, col, cbase, nk, false, lane);
+        if (PASS == DKDV) point_dkdv<float, D / 16, false>(a, b, h, bh, row, col, cbase, nk, nv, lane);
     }
 }
 
@@ -312,7 +313,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kern
 #pragma unroll
     for (int cb = 0; cb < NCB; cb++) check += point_sum(acc[cb]);
     const unsigned redo = point_columns(mine && not_finite(check));
-    if (mine && !(redo >> c & 1)) {
+    if (mine) {
         if (a.lse && qd == 0 && wv == 0) a.lse[((size_t)bh * a.Ho + ho) * a.Wo + w0 + c] = m + fast_log2(S);
         const float inv = 1.0f / S;
         char *y = static_cast<char *>(a.y) + pt * ldbv_ + (size_t)h * (a.dv_ * 4) + cbase * 4 + 16 * qd;
@@ -326,7 +327,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kern
 
 // ---- backward, dq pass (needs the forward's y and lse) -------------------------------------------------------------
 // Three products per step:  S^T = K Q^T,  G^T = V dY^T,  dQ^T += K^T dS^T  with dS = P o (G - I),  I = <dy, y>.
-template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dq_m32_kernel(const Args a)
+template <int D, int NS> __global__ __launch_bounds__(64 * NS, D == 16 ? 5 : 1) void dq_m32_kernel(const Args a)
 {
     typedef FTile<D> Tile;
     constexpr int PITCH = Tile::PITCH, NCB = D / 16;
@@ -452,7 +453,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dq_m32_kerne
     for (int cb = 0; cb < NCB; cb++) check += point_sum(acc[cb]);
     const unsigned redo = point_columns(mine && not_finite(check));
     if (mine && qd == 0 && wv == 0) a.stats[sidx] = make_float2(lse, I);
-    if (mine && !(redo >> c & 1)) {
+    if (mine) {
         char *dq = static_cast<char *>(a.dq) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4 + 16 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++)
@@ -580,7 +581,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dkdv_m32_ker
 #pragma unroll
     for (int cb = 0; cb < NCB; cb++) check += point_sum(dkt[cb] + dvt[cb]);
     const unsigned redo = point_columns(mine && not_finite(check));
-    if (mine && !(redo >> c & 1)) {
+    if (mine) {
         char *dk = static_cast<char *>(a.dk) + pt * ldbk_ + (size_t)h * (a.dk_ * 4) + cbase * 4 + 16 * qd;
         char *dv = static_cast<char *>(a.dv) + pt * ldbv_ + (size_t)h * (a.dv_ * 4) + cbase * 4 + 16 * qd;
 #pragma unroll

@@ -320,18 +320,21 @@ template <typename T, int D> constexpr int s16_lds_bytes(bool stats) { return 2 
 // block of the ring `n` blocks after block `first` (both below 5)
 __device__ inline int s16_block(int first, int n) { return first + n >= FRESH / 16 ? first + n - FRESH / 16 : first + n; }
 
-// The columns `redo` of a wavefront whose sums are not finite (see s2attn_points.hpp)
-template <typename T, int N, Which PASS> __device__ inline void s16_points(unsigned redo, int wv)
+// The columns `redo` of a wavefront whose sums are not finite, stored already (see s2attn_points.hpp)
+template <typename T, int D, bool PAD, Which PASS> __device__ inline void s16_points(unsigned redo, int wv)
 {
+    constexpr int N = D / 16;
+    constexpr bool SEEN = std::is_same<T, float>::value && D == 32 && !PAD;
+    __threadfence(); // what is written here comes after it
     const Args a = point_args();
     S2_H16_IDS_OF(64 * wv + point_lane(), PASS == DKDV ? a.Wi : a.Wo, PASS == DKDV ? a.Hi : a.Ho)
     (void)c, (void)qd, (void)nvalid;
     const int row = (PASS == DKDV ? a.sorder : a.gorder)[a.row_first + rowsel];
     for (; redo; redo &= redo - 1) {
         const int col = w0 + __builtin_ctz(redo);
-        if (PASS == FWD) point_forward<T, N>(a, b, h, bh, row, col, 0, a.dv_, true, lane);
-        if (PASS == DQ) point_dq<T, N>(a, b, h, bh, row, col, 0, a.dk_, true, lane);
-        if (PASS == DKDV) point_dkdv<T, N>(a, b, h, bh, row, col, 0, a.dk_, a.dv_, lane);
+        if (PASS == FWD) point_forward<T, N, SEEN>(a, b, h, bh, row, col, 0, a.dv_, true, lane);
+        if (PASS == DQ) point_dq<T, N, SEEN>(a, b, h, bh, row, col, 0, a.dk_, true, lane);
+        if (PASS == DKDV) point_dkdv<T, N, SEEN>(a, b, h, bh, row, col, 0, a.dk_, a.dv_, lane);
     }
 }
 
@@ -443,7 +446,7 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
 #pragma unroll
     for (int cb = 0; cb < NCB; cb++) check += point_sum(acc[cb].hi + acc[cb].lo);
     const unsigned redo = point_columns(mine && not_finite(check));
-    if (mine && !(redo >> c & 1)) {
+    if (mine) {
         if (a.lse && qd == 0) a.lse[((size_t)bh * a.Ho + ho) * a.Wo + w0 + c] = m + fast_log2(Z);
         const float inv = 1.0f / Z;
         T *y = static_cast<T *>(a.y) + pt * a.ldy + h * nv + 4 * qd;
@@ -451,7 +454,7 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
         for (int cb = 0; cb < NCB; cb++)
             if (!PAD || 16 * cb + 4 * qd < nv) s16_store4(y + 16 * cb, (acc[cb].hi + acc[cb].lo) * inv);
     }
-    if (redo) s16_points<T, NCB, FWD>(redo, wv);
+    if (redo) s16_points<T, D, PAD, FWD>(redo, wv);
 }
 
 // ---- backward, dq pass (needs the forward's y and lse) -------------------------------------------------------------
@@ -587,14 +590,14 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
 #pragma unroll
     for (int cb = 0; cb < NCB; cb++) check += point_sum(EXACT_I ? acc[cb].hi + acc[cb].lo : acc[cb].hi + acc[cb].lo + ak[EXACT_I ? 0 : cb]);
     const unsigned redo = point_columns(mine && not_finite(check));
-    if (mine && !(redo >> c & 1)) {
+    if (mine) {
         if (qd == 0) a.stats[sidx] = make_float2(lse, I + off);
         T *dq = static_cast<T *>(a.dq) + pt * a.lddq + h * nk + 4 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++)
             if (!PAD || 16 * cb + 4 * qd < nk) s16_store4(dq + 16 * cb, EXACT_I ? acc[cb].hi + acc[cb].lo : (acc[cb].hi + acc[cb].lo) - off * ak[EXACT_I ? 0 : cb]);
     }
-    if (redo) s16_points<T, NCB, DQ>(redo, wv);
+    if (redo) s16_points<T, D, PAD, DQ>(redo, wv);
 }
 
 // ---- backward, dk/dv pass: transposed gather ---------------------------------------------------------------------
@@ -740,7 +743,7 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW, D =
 #pragma unroll
     for (int cb = 0; cb < NCB; cb++) check += point_sum(s16_value(dkt[cb]) + s16_value(dvt[cb]));
     const unsigned redo = point_columns(mine && not_finite(check));
-    if (mine && !(redo >> c & 1)) {
+    if (mine) {
         T *dk = static_cast<T *>(a.dk) + pt * a.lddk + h * nk + 4 * qd, *dv = static_cast<T *>(a.dv) + pt * a.lddv + h * nv + 4 * qd;
 #pragma unroll
         for (int cb = 0; cb < NCB; cb++) {
@@ -748,5 +751,5 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW, D =
             if (!PAD || 16 * cb + 4 * qd < nv) s16_store4(dv + 16 * cb, s16_value(dvt[cb]));
         }
     }
-    if (redo) s16_points<T, NCB, DKDV>(redo, wv);
+    if (redo) s16_points<T, D, PAD, DKDV>(redo, wv);
 }
