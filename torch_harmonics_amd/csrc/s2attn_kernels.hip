@@ -2471,7 +2471,9 @@ template <typename T, int D, bool PAD, int MODE> int launch_ring_s16(const Args 
 #define S2_RING_INSTANCES(T) S2_RING_MODES(T, 32) S2_RING_MODES(T, 48) S2_RING_MODES(T, 64)
 S2_RING_INSTANCES(bf16_t)
 S2_RING_INSTANCES(f16_t)
-S2_RING_MODES(float, 48)
+template int launch_ring_s16<float, 48, true, 0>(const Args &, hipStream_t);
+template int launch_ring_s16<float, 48, true, 1>(const Args &, hipStream_t);
+template int launch_ring_s16<float, 48, true, 3>(const Args &, hipStream_t);
 template int launch_ring_s16<float, 32, true, 3>(const Args &, hipStream_t);
 template int launch_ring_s16<float, 32, false, 3>(const Args &, hipStream_t);
 #undef S2_RING_INSTANCES
@@ -3053,13 +3055,16 @@ template <int MODE, typename T> bool ring_split(const Args &a)
     const bool full = 5 * cols >= 4 * ((cols + WQ - 1) / WQ * WQ);
     if (std::is_same<T, bf16_t>::value) return true;
     if (std::is_same<T, f16_t>::value) return a.dk_ > 32 || full;
+    if (MODE == 2 || MODE == 4) return false; // (up-sampling: more than one class)
     return full && a.kps == 1 && a.r_qps == 1 && a.dk_ <= 48 && (a.dk_ > 32 || MODE == 3);
 }
 template <int MODE, typename T> int launch_ring_plan_t(const Args &a, hipStream_t st)
 {
     if (ring_split<MODE, T>(a)) {
         if constexpr (std::is_same<T, float>::value) {
-            if (a.dk_ > 32) return launch_ring_s16<T, 48, true, MODE>(a, st);
+            if constexpr (MODE == 0 || MODE == 1 || MODE == 3) {
+                if (a.dk_ > 32) return launch_ring_s16<T, 48, true, MODE>(a, st);
+            }
             if constexpr (MODE == 3) return a.dk_ == 32 ? launch_ring_s16<T, 32, false, MODE>(a, st) : launch_ring_s16<T, 32, true, MODE>(a, st);
         } else {
             if (a.dk_ <= 32) return launch_ring_s16<T, 32, true, MODE>(a, st);
