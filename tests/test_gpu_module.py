@@ -346,3 +346,51 @@ def test_module_traces_under_torch_compile():
     compiled = run(torch.compile(m, backend="aot_eager", fullgraph=True))
     for i, (e, c) in enumerate(zip(eager, compiled)):
         assert_close(f"tensor {i}", c, e, rtol=1e-6, atol=1e-6)
+
+
+COMPOSED_CASES = {
+    # B, C, heads, in_shape, out_shape, memory format, qknorm: the routes of a layer that is composed of separate operators
+    "fused_nchw": (2, 64, 2, (12, 96), (12, 96), torch.contiguous_format, False),
+    "fused_nchw_cross": (2, 64, 2, (24, 192), (12, 96), torch.contiguous_format, False),
+    "fused_many_batches": (9, 64, 2, (6, 64), (6, 64), torch.contiguous_format, False),
+    "fused_channels_last": (2, 64, 2, (12, 96), (12, 96), torch.channels_last, False),
+    "shared": (2, 24, 3, (12, 96), (12, 96), torch.contiguous_format, False),
+    "shared_channels_last": (2, 24, 3, (24, 96), (12, 48), torch.channels_last, False),
+    "qknorm": (2, 64, 2, (12, 96), (12, 96), torch.contiguous_format, True),
+}
+
+
+@pytest.mark.parametrize("case", COMPOSED_CASES)
+def test_layer_with_a_tensor_as_softmax_scale(case):
+    """A tensor as scale (here one that is trained) takes the layer apart into separate operators: output and every gradient, the
+    scale's among them, against the float64 evaluation."""
+    from torch_harmonics_amd import NeighborhoodAttentionS2
+
+    B, C, nh, ins, outs, layout, qkn = COMPOSED_CASES[case]
+    torch.manual_seed(SEED)
+    scale = torch.tensor(0.37, device=DEV, requires_grad=True)
+    m = NeighborhoodAttentionS2(C, ins, outs, num_heads=nh, use_qknorm=qkn, scale=scale, theta_cutoff=0.5).to(DEV)
+    with torch.no_grad():
+        for n, p in m.named_parameters():
+            if "bias" in n or "norm" in n:
+                p.uniform_(-0.3, 0.3)
+    xq, xk = torch.randn(B, C, *outs), torch.randn(B, C, *ins)
+    cross = ins != outs
+    gout = torch.randn(B, C, *outs)
+    dq_, dk_ = [t.to(DEV).contiguous(memory_format=layout).requires_grad_(True) for t in (xq, xk)]
+    out = m(dq_, dk_, dk_) if cross else m(dq_)
+    out.backward(gout.to(DEV))
+    rq, rk = [t.double().requires_grad_(True) for t in (xq, xk)]
+    m.scale = torch.tensor(scale.item(), dtype=torch.float64, requires_grad=True)
+    ref, params = _reference_module_forward(m, rq, rk if cross else rq, rk if cross else rq)
+    ref.backward(gout.double())
+    tol = dict(rtol=1e-4, atol=2e-5)
+    assert_close("output", out, ref, **tol)
+    assert_close("d query", dq_.grad, rq.grad, **tol)
+    if cross:
+        assert_close("d key and value", dk_.grad, rk.grad, **tol)
+    for name, prm in m.named_parameters():
+        if qkn or name != "k_bias":  # (without the norm the softmax does not see it: rounding alone)
+            bound = 1e-5 * params[name].grad.abs().max().item()  # sums over all points
+            assert_close("d " + name, prm.grad, params[name].grad, rtol=1e-4, atol=1e-4 + bound)
+    assert_close("d scale", scale.grad, m.scale.grad, rtol=1e-4, atol=1e-4 * params["q_weights"].grad.abs().sum().item() ** 0.5)

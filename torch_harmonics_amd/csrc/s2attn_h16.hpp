@@ -236,15 +236,15 @@ __device__ inline void xcd_split(int id, int BH, int per_bh, int &bh, int &rest)
     }
 }
 
-#define S2_H16_IDS(W_TILED, NROWS) S2_H16_IDS_OF(threadIdx.x, W_TILED, NROWS)
-#define S2_H16_IDS_OF(TID, W_TILED, NROWS)                                    \
+#define S2_H16_IDS(W_TILED, NROWS) S2_H16_IDS_OF(threadIdx.x, blockIdx.x, W_TILED, NROWS)
+#define S2_H16_IDS_OF(TID, BLOCK, W_TILED, NROWS)                             \
     const int tid = TID;                                                      \
     const int lane = tid & 63, wave = tid >> 6;                               \
     const int c = lane & 15, qd = lane >> 4;                                  \
     const int BH = a.B * a.nh;                                                \
     const int ntile = ((W_TILED) + WQ - 1) / WQ;                              \
     int bh, id_;                                                              \
-    xcd_split(blockIdx.x, BH, ntile *(NROWS), bh, id_);                       \
+    xcd_split(BLOCK, BH, ntile *(NROWS), bh, id_);                       \
     const int grp_ = id_ / (HG * ntile);                                      \
     const int grows_ = min(HG, (NROWS)-grp_ * HG);                            \
     id_ -= grp_ * HG * ntile;                                                 \

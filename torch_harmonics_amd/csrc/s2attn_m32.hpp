@@ -20,15 +20,15 @@
 // tiles, operands and output channels); the partial scores of the groups are added through LDS once per step, after which
 // both wavefronts hold the same probabilities.  One wavefront cannot hold a 256-channel step in registers.
 
-#define S2_M32_IDS(W_TILED, NROWS) S2_M32_IDS_OF(NS > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x, W_TILED, NROWS)
-#define S2_M32_IDS_OF(LANE, W_TILED, NROWS)                                   \
+#define S2_M32_IDS(W_TILED, NROWS) S2_M32_IDS_OF(NS > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x, NS > 1 ? (int)(threadIdx.x >> 6) : 0, blockIdx.x, W_TILED, NROWS)
+#define S2_M32_IDS_OF(LANE, WAVE, BLOCK, W_TILED, NROWS)                      \
     const int lane = LANE;                                                    \
-    const int wv = NS > 1 ? (int)(threadIdx.x >> 6) : 0;                      \
+    const int wv = WAVE;                                                      \
     const int c = lane & 15, qd = lane >> 4;                                  \
     const int BH = a.B * a.nh;                                                \
     const int ntile = ((W_TILED) + HQ - 1) / HQ;                              \
     int bh, id_;                                                              \
-    xcd_split(blockIdx.x, BH, ntile *(NROWS), bh, id_);                       \
+    xcd_split(BLOCK, BH, ntile *(NROWS), bh, id_);                       \
     const int grp_ = id_ / (HG * ntile);                                      \
     const int grows_ = min(HG, (NROWS)-grp_ * HG);                            \
     id_ -= grp_ * HG * ntile;                                                 \
@@ -177,11 +177,11 @@ template <typename T> __device__ inline u4v m32_piece(const char *p)
 }
 
 // The columns `redo` of a wavefront whose sums are not finite, stored already: its own channel group of them (see s2attn_points.hpp)
-template <int D, int NS, Which PASS> __device__ inline void m32_points(unsigned redo)
+template <int D, int NS, Which PASS> __device__ __forceinline__ void m32_points(int wave, unsigned redo)
 {
     __threadfence(); // what is written here comes after it
     const Args a = point_args();
-    S2_M32_IDS_OF(point_lane(), PASS == DKDV ? a.Wi : a.Wo, PASS == DKDV ? a.Hi : a.Ho)
+    S2_M32_IDS_OF(point_lane(), wave, blockIdx.x, PASS == DKDV ? a.Wi : a.Wo, PASS == DKDV ? a.Hi : a.Ho)
     (void)c, (void)qd, (void)nvalid, (void)ldbk_, (void)ldbv_;
     const int row = (PASS == DKDV ? a.sorder : a.gorder)[a.row_first + rowsel];
     for (; redo; redo &= redo - 1) {
@@ -322,7 +322,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void fwd_m32_kern
             if (16 * cb + 4 * qd < nv)
                 *reinterpret_cast<float4 *>(y + 64 * cb) = make_float4(acc[cb][0] * inv, acc[cb][1] * inv, acc[cb][2] * inv, acc[cb][3] * inv);
     }
-    if (redo) m32_points<D, NS, FWD>(redo);
+    if (__builtin_expect(redo != 0, 0)) m32_points<D, NS, FWD>(__builtin_amdgcn_readfirstlane(wv), redo);
 }
 
 // ---- backward, dq pass (needs the forward's y and lse) -------------------------------------------------------------
@@ -459,7 +459,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS, D == 16 ? 5 : 1) 
         for (int cb = 0; cb < NCB; cb++)
             if (16 * cb + 4 * qd < nk) *reinterpret_cast<float4 *>(dq + 64 * cb) = make_float4(acc[cb][0], acc[cb][1], acc[cb][2], acc[cb][3]);
     }
-    if (redo) m32_points<D, NS, DQ>(redo);
+    if (__builtin_expect(redo != 0, 0)) m32_points<D, NS, DQ>(__builtin_amdgcn_readfirstlane(wv), redo);
 }
 
 // ---- backward, dk/dv pass: transposed gather ---------------------------------------------------------------------
@@ -590,7 +590,7 @@ template <int D, int NS> __global__ __launch_bounds__(64 * NS) void dkdv_m32_ker
             if (16 * cb + 4 * qd < nv) *reinterpret_cast<float4 *>(dv + 64 * cb) = make_float4(dvt[cb][0], dvt[cb][1], dvt[cb][2], dvt[cb][3]);
         }
     }
-    if (redo) m32_points<D, NS, DKDV>(redo);
+    if (__builtin_expect(redo != 0, 0)) m32_points<D, NS, DKDV>(__builtin_amdgcn_readfirstlane(wv), redo);
 }
 
 // ---- forward, one ring step --------------------------------------------------------------------------------------

@@ -17,19 +17,26 @@
 // Lane l = (j = l % 16, g = l / 16): four neighbors at a time, the lanes of a group share one neighbor's channels (j, j + 16, ...).
 // Bound by the latency of the loads: about ten times slower than the tiles where everything is NaN.
 
-// The arguments of the running kernel and the lane's index, made anew: kept in registers through the walk, what the tail computes
-// from them cost the 16-channel forward one of its five wavefronts per SIMD.
+// The evaluation reads the arguments of the kernel again and counts the lanes anew, so nothing is kept in registers through a walk for it
+// (kept there, it cost the 16-channel forward one of its five wavefronts per SIMD), and stands behind the end of its kernel (among the
+// blocks of the walk it cost the 16-channel fp32 tiles 2 %).
 __device__ inline Args point_args()
 {
-    const int *p = (const int *)__builtin_amdgcn_kernarg_segment_ptr();
-    asm("" : "+s"(p));
+    typedef const int __attribute__((address_space(4))) * words;
+    words p = (words)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
     Args a;
     static_assert(sizeof(Args) % 4 == 0, "read as 32-bit words");
 #pragma unroll
-    for (unsigned i = 0; i < sizeof(Args) / 4; i++) reinterpret_cast<int *>(&a)[i] = uniform_load(p + i);
+    for (unsigned i = 0; i < sizeof(Args) / 4; i++) reinterpret_cast<int *>(&a)[i] = p[i];
     return a;
 }
-__device__ inline int point_lane() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+__device__ inline int point_lane()
+{
+    unsigned zero = 0;
+    asm volatile("" : "+s"(zero));
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
 
 // Columns (bits 0 .. 15) in which any of the four lanes of the column says so
 __device__ inline unsigned point_columns(bool any)

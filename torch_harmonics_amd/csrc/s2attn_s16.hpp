@@ -321,13 +321,13 @@ template <typename T, int D> constexpr int s16_lds_bytes(bool stats) { return 2 
 __device__ inline int s16_block(int first, int n) { return first + n >= FRESH / 16 ? first + n - FRESH / 16 : first + n; }
 
 // The columns `redo` of a wavefront whose sums are not finite, stored already (see s2attn_points.hpp)
-template <typename T, int D, bool PAD, Which PASS> __device__ inline void s16_points(unsigned redo, int wv)
+template <typename T, int D, bool PAD, Which PASS> __device__ __forceinline__ void s16_points(int wv, unsigned redo)
 {
     constexpr int N = D / 16;
     constexpr bool SEEN = std::is_same<T, float>::value && D == 32 && !PAD;
     __threadfence(); // what is written here comes after it
     const Args a = point_args();
-    S2_H16_IDS_OF(64 * wv + point_lane(), PASS == DKDV ? a.Wi : a.Wo, PASS == DKDV ? a.Hi : a.Ho)
+    S2_H16_IDS_OF(64 * wv + point_lane(), blockIdx.x, PASS == DKDV ? a.Wi : a.Wo, PASS == DKDV ? a.Hi : a.Ho)
     (void)c, (void)qd, (void)nvalid;
     const int row = (PASS == DKDV ? a.sorder : a.gorder)[a.row_first + rowsel];
     for (; redo; redo &= redo - 1) {
@@ -454,7 +454,7 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
         for (int cb = 0; cb < NCB; cb++)
             if (!PAD || 16 * cb + 4 * qd < nv) s16_store4(y + 16 * cb, (acc[cb].hi + acc[cb].lo) * inv);
     }
-    if (redo) s16_points<T, D, PAD, FWD>(redo, wv);
+    if (__builtin_expect(redo != 0, 0)) s16_points<T, D, PAD, FWD>(wv, redo);
 }
 
 // ---- backward, dq pass (needs the forward's y and lse) -------------------------------------------------------------
@@ -597,7 +597,7 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW) voi
         for (int cb = 0; cb < NCB; cb++)
             if (!PAD || 16 * cb + 4 * qd < nk) s16_store4(dq + 16 * cb, EXACT_I ? acc[cb].hi + acc[cb].lo : (acc[cb].hi + acc[cb].lo) - off * ak[EXACT_I ? 0 : cb]);
     }
-    if (redo) s16_points<T, D, PAD, DQ>(redo, wv);
+    if (__builtin_expect(redo != 0, 0)) s16_points<T, D, PAD, DQ>(wv, redo);
 }
 
 // ---- backward, dk/dv pass: transposed gather ---------------------------------------------------------------------
@@ -751,5 +751,5 @@ template <typename T, int D, bool PAD> __global__ __launch_bounds__(64 * NW, D =
             if (!PAD || 16 * cb + 4 * qd < nv) s16_store4(dv + 16 * cb, s16_value(dvt[cb]));
         }
     }
-    if (redo) s16_points<T, D, PAD, DKDV>(redo, wv);
+    if (__builtin_expect(redo != 0, 0)) s16_points<T, D, PAD, DKDV>(wv, redo);
 }
