@@ -186,9 +186,9 @@ template <int D, int NS, Which PASS> __device__ __forceinline__ void m32_points(
     const int row = (PASS == DKDV ? a.sorder : a.gorder)[a.row_first + rowsel];
     for (; redo; redo &= redo - 1) {
         const int col = w0 + __builtin_ctz(redo);
-        if (PASS == FWD) point_forward<float, D / 16, false>(a, b, h, bh, row, col, cbase, nv, wv == 0, lane);
-        if (PASS == DQ) point_dq<float, D / 16, false>(a, b, h, bh, row, col, cbase, nk, false, lane);
-        if (PASS == DKDV) point_dkdv<float, D / 16, false>(a, b, h, bh, row, col, cbase, nk, nv, lane);
+        if (PASS == FWD) point_forward<float, D / 16, NS * D / 16, false>(a, b, h, bh, row, col, cbase, nv, wv == 0, lane);
+        if (PASS == DQ) point_dq<float, D / 16, NS * D / 16, false>(a, b, h, bh, row, col, cbase, nk, false, lane);
+        if (PASS == DKDV) point_dkdv<float, D / 16, NS * D / 16, false>(a, b, h, bh, row, col, cbase, nk, nv, lane);
     }
 }
 

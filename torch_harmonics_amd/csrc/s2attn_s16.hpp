@@ -332,9 +332,9 @@ template <typename T, int D, bool PAD, Which PASS> __device__ __forceinline__ vo
     const int row = (PASS == DKDV ? a.sorder : a.gorder)[a.row_first + rowsel];
     for (; redo; redo &= redo - 1) {
         const int col = w0 + __builtin_ctz(redo);
-        if (PASS == FWD) point_forward<T, N, SEEN>(a, b, h, bh, row, col, 0, a.dv_, true, lane);
-        if (PASS == DQ) point_dq<T, N, SEEN>(a, b, h, bh, row, col, 0, a.dk_, true, lane);
-        if (PASS == DKDV) point_dkdv<T, N, SEEN>(a, b, h, bh, row, col, 0, a.dk_, a.dv_, lane);
+        if (PASS == FWD) point_forward<T, N, N, SEEN>(a, b, h, bh, row, col, 0, a.dv_, true, lane);
+        if (PASS == DQ) point_dq<T, N, N, SEEN>(a, b, h, bh, row, col, 0, a.dk_, true, lane);
+        if (PASS == DKDV) point_dkdv<T, N, N, SEEN>(a, b, h, bh, row, col, 0, a.dk_, a.dv_, lane);
     }
 }
 
