@@ -7,7 +7,7 @@
 // current stream.  There is no CPU implementation: CPU tensors are refused with a clear error.
 //
 // s2attn_kernels::module_attention is the whole NeighborhoodAttentionS2 layer (projections, q/k norm, attention, output projection)
-// as ONE autograd node: eleven launches per training step and no Python between them, where the operator-by-operator form
+// as ONE autograd node: twelve launches per training step (self-attention without q/k norm) and no Python between them, where the operator-by-operator form
 // needs about forty and spends 0.8 ms of host time on them.
 //
 // Built by the Makefile next to it into torch_harmonics_amd/_C.so and loaded with torch.ops.load_library; the fake (meta)
