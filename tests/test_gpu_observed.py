@@ -187,6 +187,7 @@ def test_opcheck_of_the_layer(layer):
     m, xs = layer
     args = _layer_args(m, [x.requires_grad_() for x in xs], xs[0].dtype)
     torch.library.opcheck(ops.layer_forward, (*args, True))
+    torch.library.opcheck(ops.layer_forward, args)  # (the flag's default)
     plain = tuple(a.detach() if isinstance(a, torch.Tensor) else a for a in args)
     torch.library.opcheck(ops.layer_forward, (*plain, False))
     out, *kept = ops.layer_forward(*plain, True)

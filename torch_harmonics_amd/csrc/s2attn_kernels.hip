@@ -61,7 +61,7 @@ int s2attn_fail(int code, const char *fmt, ...)
 }
 
 extern "C" const char *s2attn_last_error(void) { return g_err; }
-extern "C" int s2attn_abi_version(void) { return 13; }
+extern "C" int s2attn_abi_version(void) { return 14; }
 #endif
 
 namespace s2 {

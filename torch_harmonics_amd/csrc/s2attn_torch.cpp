@@ -852,7 +852,7 @@ TORCH_LIBRARY(s2attn_kernels, m)
         "Tensor? v_bias, Tensor? proj_bias, Tensor? q_norm, Tensor? k_norm, float scale, Tensor quad_weights, Tensor col_idx, Tensor row_off, Tensor plan, "
         "int[] plan_header, int num_heads, int nlat_in, int nlon_in, int nlat_out, int nlon_out, ScalarType compute";
     m.def(("module_attention(" + layer + ") -> Tensor").c_str(), &module_attention);
-    m.def(("layer_forward(" + layer + ", bool keep) -> Tensor[]").c_str(), {at::Tag::pt2_compliant_tag});
+    m.def(("layer_forward(" + layer + ", bool keep=True) -> Tensor[]").c_str(), {at::Tag::pt2_compliant_tag});
     std::string thirteen = "Tensor";
     for (int i = 1; i < NGRADS; i++) thirteen += ", Tensor";
     m.def(("layer_backward(Tensor grad, " + layer + ", Tensor q, Tensor k, Tensor v, Tensor q_raw, Tensor k_raw, Tensor y, Tensor lse, bool[13] need) -> (" + thirteen + ")").c_str(), {at::Tag::pt2_compliant_tag});

@@ -274,7 +274,7 @@ _LAYER_TENSORS = 13  # query, key, value, four weights, four biases, two norm ga
 
 @torch.library.register_fake("s2attn_kernels::layer_forward")
 def _(query, key, value, q_weights, k_weights, v_weights, proj_weights, q_bias, k_bias, v_bias, proj_bias, q_norm, k_norm, scale, quad_weights, col_idx,
-      row_off, plan, plan_header, num_heads, nlat_in, nlon_in, nlat_out, nlon_out, compute, keep):  # fmt: skip
+      row_off, plan, plan_header, num_heads, nlat_in, nlon_in, nlat_out, nlon_out, compute, keep=True):  # fmt: skip
     B, ck, cv = query.shape[0], q_weights.shape[0], v_weights.shape[0]
     new = lambda *s: query.new_empty(s, dtype=compute)  # noqa: E731
     if not keep:
@@ -295,7 +295,7 @@ def _(grad, *args):
 
 def _layer_setup_context(ctx, inputs, output):
     ctx.save_for_backward(*inputs[:_LAYER_TENSORS], *inputs[14:18], *output[1:])
-    ctx.scale, ctx.rest, ctx.kept = inputs[13], inputs[18:-1], inputs[-1]
+    ctx.scale, ctx.rest, ctx.kept, ctx.ninputs = inputs[13], inputs[18:25], all(inputs[25:]), len(inputs)
     ctx.set_materialize_grads(False)
 
 
@@ -303,12 +303,12 @@ def _layer_backward_rule(ctx, grads):
     saved = ctx.saved_tensors
     tensors, geometry, kept = saved[:_LAYER_TENSORS], saved[_LAYER_TENSORS : _LAYER_TENSORS + 4], saved[_LAYER_TENSORS + 4 :]
     if grads[0] is None:
-        return (None,) * (_LAYER_TENSORS + 13)
+        return (None,) * ctx.ninputs
     if not ctx.kept:
         raise RuntimeError("layer_forward ran with keep=False: nothing of it is left for a backward")
     need = [t is not None and bool(n) for t, n in zip(tensors, ctx.needs_input_grad)]
     out = layer_backward(grads[0], *tensors, ctx.scale, *geometry, *ctx.rest, *kept, need)
-    return (*[g if n else None for g, n in zip(out, need)], *(None,) * 13)
+    return (*[g if n else None for g, n in zip(out, need)], *(None,) * (ctx.ninputs - _LAYER_TENSORS))
 
 
 def _no_second_derivative(ctx, *grads):
