@@ -295,7 +295,8 @@ def _(grad, *args):
 
 def _layer_setup_context(ctx, inputs, output):
     ctx.save_for_backward(*inputs[:_LAYER_TENSORS], *inputs[14:18], *output[1:])
-    ctx.scale, ctx.rest, ctx.kept, ctx.ninputs = inputs[13], inputs[18:25], all(inputs[25:]), len(inputs)
+    ctx.scale, ctx.rest, ctx.kept = inputs[13], inputs[18:25], all(inputs[25:])
+    ctx.ninputs = 25 if ctx.kept else 26  # (an argument at its default does not count)
     ctx.set_materialize_grads(False)
 
 
