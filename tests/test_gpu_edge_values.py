@@ -21,6 +21,9 @@ pytestmark = pytest.mark.gpu
 SHAPES = {
     "f32_c3c5": (F32, 3, 5, (9, 48), 1, 2, "vector"),
     "f32_c8": (F32, 8, 8, (9, 48), 1, 2, "fp32"),
+    "f32_c4_w96": (F32, 4, 4, (9, 96), 1, 2, "fp32"),
+    "f32_c8_w96": (F32, 8, 8, (9, 96), 1, 2, "fp32"),
+    "f32_c12_w96_many": (F32, 12, 12, (9, 96), 30, 2, "split"),
     "f32_c8_many": (F32, 8, 8, (9, 48), 60, 2, "split"),
     "f32_c4c12_many": (F32, 4, 12, (9, 48), 60, 2, "split"),
     "f32_c16_many": (F32, 16, 16, (9, 48), 60, 2, "split"),
